@@ -4,9 +4,11 @@
 //   s16     mamba2_recall/state_codec.py:65-102 (_s16_scan)
 //
 // A translation unit of its own: it is compiled with the default machine
-// scheduler, the dense3 and packed-row steps with the max-ILP one.
+// scheduler, the dense3 and packed-row steps and the row-split scans
+// (m2r_rows.hip) with the max-ILP one.
 #include "m2r_device.h"
 #include "m2r_abi_util.h"
+#include "m2r_rows.h"
 #include "m2r_tile.h"
 
 namespace m2r {
@@ -20,14 +22,6 @@ namespace m2r {
 // sub-tile as (r0 + r1) + (r2 + r3) (the per-program tl.sum of :102), and
 // the four sub-tiles of a 16-row tile in order, ((T0 + T1) + T2) + T3 (the
 // host-side sum of state_codec.py:255-261).
-struct S16Args {
-  const uint16_t* x; const uint16_t* dt; const float* A; const uint16_t* Bm; const uint16_t* Cm;
-  const void* D; const void* dt_bias;
-  uint16_t* state; uint16_t* y; float* stats;
-  int B, L, H, P, G;
-  int d_f32, db_f32;
-};
-
 // STAGED (state 16-byte aligned): the slot's 64 rows of 256 B move between
 // HBM and registers through LDS, one half-row (128 B) of every row at a
 // time, as 1 KiB wave-wide transfers (8 per half, each 8 rows x 128 B);
@@ -180,6 +174,18 @@ extern "C" int m2r_state_step_s16(const void* x, const void* dt, const float* A,
                db_is_f32};
   const dim3 grid((unsigned)((P + 63) / 64), (unsigned)H, (unsigned)batch);
   const bool staged = ((uintptr_t)state & 15) == 0;
+  // Several tokens: eight lanes per row, where rows, inputs and readouts are
+  // whole 16-byte pieces.  Without statistics, a call of many rows and few
+  // tokens mostly streams its carry, which one lane per row does better: us
+  // per call, one lane / eight lanes, at batch 4 (512 slots of 64 rows) 13.7 /
+  // 9.6 for 2 tokens; batch 16 (2,048) 20.9 / 30.1 for 2, 45.0 / 44.5 for 8;
+  // batch 64 (8,192) 66 / 99 for 2, 124 / 149 for 8, 393 / 389 for 32.  With
+  // statistics, whose per-row sums the one-lane form keeps in LDS, eight lanes
+  // are faster throughout (batch 64, 2 tokens: 208 / 123).
+  const long long slots = (long long)batch * H * ((P + 63) / 64);
+  if (L > 1 && (stats || 256 * L >= slots) && P % 8 == 0 && staged &&
+      (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C | (uintptr_t)y) & 15) == 0)
+    return m2r_check(launch_s16_rows(args, stream), "s16 step launch");
   if (staged && stats) hipLaunchKernelGGL((k_s16_step<true, true>), grid, dim3(64), 0, stream, args);
   else if (staged) hipLaunchKernelGGL((k_s16_step<true, false>), grid, dim3(64), 0, stream, args);
   else if (stats) hipLaunchKernelGGL((k_s16_step<false, true>), grid, dim3(64), 0, stream, args);

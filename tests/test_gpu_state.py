@@ -683,6 +683,15 @@ def test_s16_control_step(oracle, device):
     run_s16(oracle, device, 2, 7, 32, 64, 4, 83, collect=True)      # whole tiles, several tokens
 
 
+@pytest.mark.parametrize("batch,L,H,P,G", [(1, 2, 8, 8, 8), (2, 31, 16, 24, 2), (1, 33, 8, 40, 4), (1, 64, 4, 64, 1),
+                                           (1, 97, 6, 72, 3), (3, 130, 4, 16, 2)])
+@pytest.mark.parametrize("collect", [False, True])
+def test_s16_rows_block_edges(oracle, device, batch, L, H, P, G, collect):
+    """The row-split multi-token scan around its 32-token blocks, its 64-token
+    dt batches and its 32-row workgroups (P down to one wave's 8 rows)."""
+    run_s16(oracle, device, batch, L, H, P, G, 8800 + L, collect)
+
+
 def test_s16_statistics_same_on_every_run(oracle, device):
     """The statistics feed a stable argsort of per-coordinate means
     (scripts/run_statequant.py:83): the same data must give the same bits on
