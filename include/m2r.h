@@ -55,12 +55,13 @@ int m2r_state_step_ridge(const void* x, const void* dt, const float* A, const vo
  * The same step with a caller workspace for its token records.  The
  * reference computes the ridge correction of every token's readout weights
  * before its scan (scripts/fp4_zero_predictor_codec_v1.py:221-225, the einsum
- * over all L tokens); here, for L > 1 on the small-batch shapes (at most 1024
- * 64-row slots) with 16-byte transfers, a first kernel writes one record per
- * (batch row, token, group) of the state-independent token values (readout
- * weights with the correction, dead-tier dot products, sum b.c, the carried
- * b) into `workspace`, and the scan reads them instead of building each token
- * itself.  Results are identical to m2r_state_step_ridge bit for bit.
+ * over all L tokens); here, for L > 1 with 16-byte transfers and 16-byte
+ * aligned x, B, C and y, a first kernel writes one record per (batch row, token, group) of the
+ * state-independent token values (readout weights with the correction,
+ * dead-tier dot products, sum b.c, the carried b) into `workspace`, and the
+ * multi-token scan, which spreads each row over one to eight lanes, reads
+ * them (faster from 16 to 64 tokens on, by the number of rows).  Results are
+ * identical to m2r_state_step_ridge bit for bit.
  * workspace: null (then exactly m2r_state_step_ridge), or 16-byte aligned
  * device memory of at least m2r_ridge_records_bytes(batch, L, G) bytes,
  * used on `stream` only (calls that overlap on one workspace race).
@@ -102,7 +103,8 @@ int m2r_state_step_legacy(const void* x, const void* dt, const float* A, const v
  * automatic choice at small batches), or (4,-4): four waves, all on one head
  * slot (each wave steps a quarter of the carried coordinates); (0,0) restores
  * the automatic choice.  A forced shape whose head count does not divide the heads per group
- * falls back to the automatic choice.  Process-wide; results do not depend on the shape.  No counterpart
+ * falls back to the automatic choice.  A forced shape also keeps multi-token calls on the one-lane-per-row
+ * kernels, except (4,0), (4,-2) and (4,-4) with a ridge workspace.  Process-wide; results do not depend on the shape.  No counterpart
  * in the reference (its Triton launch grid is fixed per call).
  */
 int m2r_set_step_shape(int waves_per_block, int heads_per_wave);

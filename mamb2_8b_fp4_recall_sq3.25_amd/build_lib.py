@@ -4,7 +4,7 @@ Every translation unit is compiled with binary32 contraction disabled
 (-ffp-contract=off: the codec's bit-exactness relies on separately rounded
 products and sums), IEEE denormals kept, and packed-FP32 instruction
 selection disabled.  The packed-row and dense3 step kernels (m2r_state.hip,
-the instrumented copy that includes it, m2r_dense3.hip, m2r_rows.hip) are
+the instrumented copy that includes it, m2r_dense3.hip, m2r_rows*.hip) are
 scheduled for instruction-level parallelism (SOURCE_FLAGS).  Objects are compiled in
 parallel, then linked.
 """
@@ -41,7 +41,8 @@ FLAGS = [
 # slower with it.
 SCHED_ILP_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 SOURCE_FLAGS = {"m2r_state.hip": SCHED_ILP_FLAGS, "m2r_timeline.hip": SCHED_ILP_FLAGS,
-                "m2r_dense3.hip": SCHED_ILP_FLAGS, "m2r_rows.hip": SCHED_ILP_FLAGS}
+                "m2r_dense3.hip": SCHED_ILP_FLAGS, "m2r_rows.hip": SCHED_ILP_FLAGS,
+                "m2r_rows_ridge.hip": SCHED_ILP_FLAGS}
 
 
 def sources():

@@ -14,6 +14,8 @@
 // max(RN(amax_half / 3), 1e-8) through the exact reciprocal-form quotient.
 #include "m2r_device.h"
 #include "m2r_abi_util.h"
+#include "m2r_rows.h"
+#include "m2r_step.h"
 #include "m2r_tile.h"
 
 #include <type_traits>
@@ -680,6 +682,16 @@ extern "C" int m2r_state_step_dense3(const void* x, const void* dt, const float*
     const long long slots = (long long)batch * H * pblocks;
     int wpb = 1, hpw = 1;
     const int forced = m2r_forced_step_shape();
+    // several tokens: the row-split scan where it pays (16-byte pieces)
+    if (L > 1 && !forced && rows_scan_pays(MODE_DENSE3, 128, slots, (int)L) && P % 8 == 0 &&
+        (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C | (uintptr_t)y) & 15) == 0) {
+      StepArgs r{};
+      r.x = args.x; r.dt = args.dt; r.A = A; r.Bm = args.Bm; r.Cm = args.Cm; r.D = D; r.dt_bias = dt_bias;
+      r.perm = (const uint8_t*)table; r.lo = codes; r.s8 = args.scales; r.y = args.y;
+      r.B = args.B; r.L = args.L; r.H = args.H; r.P = args.P; r.G = args.G;
+      r.d_f32 = d_is_f32; r.db_f32 = db_is_f32;
+      return m2r_check(launch_dense3_rows(r, table_is_equalizer, stream), "dense3 step launch");
+    }
     if (forced && (forced & 15) && hpg % ((forced >> 4) * (forced & 15)) == 0 && (forced >> 4) != 8) {
       wpb = forced >> 4;
       hpw = forced & 15;

@@ -1,12 +1,12 @@
 // Multi-token scans with each state row spread over several lanes, for gfx950.
 //
 //   s16     mamba2_recall/state_codec.py:65-102 (_s16_scan)
+//   dense3, tier, legacy: m2r_rows_kernel.h
 //
 // Compiled with the max-ILP machine scheduler: 180 -> 167 us for 512 tokens
 // of the FP16 carry at batch 1, against the default one.
-#include "m2r_device.h"
+#include "m2r_rows_kernel.h"
 #include "m2r_rows.h"
-#include "m2r_tile.h"
 
 namespace m2r {
 
@@ -180,6 +180,39 @@ hipError_t launch_s16_rows(const S16Args& a, hipStream_t stream) {
   if (a.stats) hipLaunchKernelGGL((k_s16_rows<true>), grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((k_s16_rows<false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
+}
+
+// The scan pays its taking apart and putting together of the rows with the
+// first tokens.  us per call, one lane per row / this scan, at batch 1, 8 and
+// 64 (128, 1,024 and 8,192 slots):
+//   tier 32/32/64     8 tokens 14.4 / 11.3, 20.5 / 20.7, 102.2 / 115.7
+//                    16 tokens 24.0 / 14.8, 33.4 / 30.5, 183.1 / 180.5
+//   legacy 16/64/48   8 tokens 14.6 / 12.4, 22.2 / 23.0, 136.6 / 150.6
+//   dense3            2 tokens 11.9 /  9.2,  4: 22.2 / 20.6, 16: 299.9 / 280.2
+// Wide rows over many slots (four lanes per row, see rows_lanes) come out
+// even near 64 tokens: tier 8/80/40 at batch 16, 222.0 / 221.0.
+// (A ridge scan runs where its caller brings a workspace.)
+bool rows_scan_pays(int mode, int carried, long long slots, int L) {
+  if (mode == MODE_DENSE3) return L >= (slots <= 384 ? 2 : slots <= 1024 ? 4 : 16);
+  if (slots > 1024 && carried > 72) return L >= 64;
+  return L >= (slots <= 384 ? 8 : slots <= 1024 ? 16 : 24);
+}
+
+template <int N8, int N4, int NZ, int MODE>
+hipError_t launch_rows(const StepArgs& a, hipStream_t stream) {
+  return launch_rows_scan<N8, N4, NZ, MODE>(a, 0, stream);
+}
+template hipError_t launch_rows<16, 64, 48, MODE_LEGACY>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<16, 64, 48, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<8, 80, 40, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<24, 48, 56, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<32, 32, 64, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<36, 24, 68, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<40, 16, 72, MODE_STORED>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<44, 8, 76, MODE_STORED>(const StepArgs&, hipStream_t);
+
+hipError_t launch_dense3_rows(const StepArgs& a, int equalizer, hipStream_t stream) {
+  return launch_rows_scan<64, 64, 0, MODE_DENSE3>(a, equalizer, stream);
 }
 
 }  // namespace m2r

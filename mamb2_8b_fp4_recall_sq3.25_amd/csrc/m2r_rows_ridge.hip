@@ -1,0 +1,22 @@
+// The row-split multi-token scan of ridge-latent rows (m2r_rows_kernel.h),
+// behind the kernel that writes its token records.
+#include "m2r_rows_kernel.h"
+#include "m2r_rows.h"
+
+namespace m2r {
+
+template <int N8, int N4, int NZ, int MODE>
+hipError_t launch_rows(const StepArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL((k_token_records<N8, N4, NZ>), dim3((a.L + REC_TOKENS - 1) / REC_TOKENS, a.G, a.B), dim3(256), 0,
+                     stream, a, (float*)a.rec);
+  return launch_rows_scan<N8, N4, NZ, MODE>(a, 0, stream);
+}
+template hipError_t launch_rows<36, 20, 72, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<16, 60, 52, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<32, 28, 68, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<40, 12, 76, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<24, 44, 60, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<8, 76, 44, MODE_RIDGE>(const StepArgs&, hipStream_t);
+template hipError_t launch_rows<44, 4, 80, MODE_RIDGE>(const StepArgs&, hipStream_t);
+
+}  // namespace m2r

@@ -1,6 +1,7 @@
 // Host dispatch and C ABI of the fused state step (kernel in m2r_step.h).
 #include "m2r_step.h"
 #include "m2r_abi_util.h"
+#include "m2r_rows.h"
 
 #include <atomic>
 #include <type_traits>
@@ -28,13 +29,6 @@ static constexpr int FOUR_PER_SLOT = 256 + 4 * 16;
 template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, int WPS = 1>
 static void launch_shape(const StepArgs& a, dim3 grid, hipStream_t stream) {
   constexpr bool staged = StepSmem<N8, N4, NZ, MODE, WPB, HPW, true, true, WPS>::STAGED;
-  if constexpr (MODE == MODE_RIDGE && WPS > 1) {   // the record-fed instance (a.rec: records written)
-    if (a.rec) {
-      hipLaunchKernelGGL((k_state_step<N8, N4, NZ, MODE, WPB, HPW, true, false, WPS, true>), grid, dim3(64 * WPB), 0,
-                         stream, a);
-      return;
-    }
-  }
   if ((a.dma_tiles & 1) && a.L == 1 && (!staged || (a.dma_tiles & 2))) {
     hipLaunchKernelGGL((k_state_step<N8, N4, NZ, MODE, WPB, HPW, true, true, WPS>), grid, dim3(64 * WPB), 0, stream,
                        a);
@@ -47,11 +41,8 @@ static void launch_shape(const StepArgs& a, dim3 grid, hipStream_t stream) {
   }
 }
 
-// args.rec on entry: a token-record workspace of at least B * L * G records
-// (or null).  The shapes of several waves per slot take it for a
-// multi-token ridge launch with 16-byte transfers: k_token_records fills it
-// and the step's token loop reads the records instead of building each
-// token (the same values); every other launch runs with rec = null.
+// args.rec: a token-record workspace of at least B * L * G records (or
+// null), for the row-split scan of a multi-token ridge launch.
 template <int N8, int N4, int NZ, int MODE>
 static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   StepArgs a = args;
@@ -60,25 +51,21 @@ static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   const int hpg = a.H / a.G;
   const long long slots = (long long)a.B * a.H * pblocks;
   const int forced = g_forced_shape.load(std::memory_order_relaxed);
-  float* const ws = (float*)args.rec;
-  a.rec = nullptr;
-  // the token records of a shape of several waves per slot
-  auto records = [&]() {
-    if constexpr (MODE == MODE_RIDGE) {
-      if (ws && a.L > 1 && (a.dma_tiles & 1)) {
-        hipLaunchKernelGGL((k_token_records<N8, N4, NZ>), dim3((a.L + REC_TOKENS - 1) / REC_TOKENS, a.G, a.B),
-                           dim3(256), 0, stream, a, ws);
-        a.rec = ws;
-      }
-    }
-  };
+  // Several tokens: the row-split scan, where rows, inputs and readouts are
+  // whole 16-byte pieces: a ridge launch that brings a workspace for its token
+  // records, another where the scan pays (m2r_rows.hip).  A forced shape keeps
+  // it away, but the shapes of several waves per slot take token records.
+  const bool rows_ok = a.L > 1 && (a.dma_tiles & 1) &&
+                       (((uintptr_t)a.x | (uintptr_t)a.Bm | (uintptr_t)a.Cm | (uintptr_t)a.y) & 15) == 0;
+  const bool rows = MODE == MODE_RIDGE ? a.rec && (!forced || forced == 4 * 16 || forced == FOUR_PER_SLOT)
+                                       : !forced && rows_scan_pays(MODE, N8 + N4, slots, a.L);
+  if (rows_ok && rows)
+    return launch_rows<N8, N4, NZ, MODE>(a, stream);
   if (forced == 4 * 16 && hpg % 2 == 0) {   // (4, 0): two waves per head slot
-    records();
     launch_shape<N8, N4, NZ, MODE, 4, 1, 2>(a, dim3(pblocks, a.H / 2, a.B), stream);
     return hipGetLastError();
   }
   if (forced == FOUR_PER_SLOT) {   // (4, -4): four waves per head slot
-    records();
     launch_shape<N8, N4, NZ, MODE, 4, 1, 4>(a, dim3(pblocks, a.H, a.B), stream);
     return hipGetLastError();
   }
@@ -95,10 +82,8 @@ static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   if (hpg % 16 == 0 && slots >= 16LL * 512) {
     launch_shape<N8, N4, NZ, MODE, 4, 4>(a, dim3(pblocks, a.H / 16, a.B), stream);
   } else if (slots <= 512) {   // four waves per slot, up to two waves per SIMD
-    records();
     launch_shape<N8, N4, NZ, MODE, 4, 1, 4>(a, dim3(pblocks, a.H, a.B), stream);
   } else if (hpg % 2 == 0 && slots <= 1024) {   // two waves per slot, up to two waves per SIMD
-    records();
     launch_shape<N8, N4, NZ, MODE, 4, 1, 2>(a, dim3(pblocks, a.H / 2, a.B), stream);
   } else if (hpg % 8 == 0 && slots >= 8LL * 512) {
     launch_shape<N8, N4, NZ, MODE, 4, 2>(a, dim3(pblocks, a.H / 8, a.B), stream);

@@ -31,7 +31,7 @@
 
 namespace m2r {
 
-enum { MODE_LEGACY = 0, MODE_STORED = 1, MODE_RIDGE = 2 };
+enum { MODE_LEGACY = 0, MODE_STORED = 1, MODE_RIDGE = 2, MODE_DENSE3 = 3 };   // (dense3: m2r_rows_kernel.h only)
 
 // Phase timeline of one launch, compiled only into the instrumented build
 // (M2R_PHASE_TIMELINE; the library proper has none of it).  Lane 0 of every
@@ -42,15 +42,11 @@ enum { MODE_LEGACY = 0, MODE_STORED = 1, MODE_RIDGE = 2 };
 // which gives the shader clock's rate.  Phases of slot k (k < 4) are stamps
 // ST_SLOT + 4 k + {0: its data landed, 1: update (one wave per slot: INT8
 // tier) done, 2: barrier passed (one wave per slot: INT4 tier done), 3: slot
-// done}.  Multi-token launches of several waves per slot also stamp token
-// ST_TL_TOKEN at ST_TL + {0: token start, 1: token values ready (record read
-// or token built), 2: update half done, 3: maxima barrier passed, 4:
-// requantization half done, 5: token end}.
+// done}.
 enum {
   ST_START = 0, ST_ARGS = 1, ST_ISSUED = 2, ST_SLOT0_ISSUED = 3, ST_ACT = 4, ST_TOKEN = 5, ST_BARRIER = 6,
-  ST_BUILD = 7, ST_SLOT = 8, ST_TL = 12, ST_COPYOUT = 24, ST_END = 25, ST_REAL0 = 30, ST_REAL1 = 31
+  ST_BUILD = 7, ST_SLOT = 8, ST_COPYOUT = 24, ST_END = 25, ST_REAL0 = 30, ST_REAL1 = 31
 };
-constexpr int ST_TL_TOKEN = 100;
 #ifdef M2R_PHASE_TIMELINE
 __device__ unsigned long long* g_phase_stamps;
 #define M2R_STAMP(i)                                                                     \
@@ -94,9 +90,9 @@ struct StepArgs {
                            // even and 4-byte aligned x, dt, A, D, dt_bias, perm (and basis): the
                            // one-token instances may stage their inputs by dword transfers
   float rhpg;              // 1 / (H / G) rounded to binary32: group of head h = (int)((h + 0.5) * rhpg)
-  // multi-token ridge launches of several waves per slot: the token records
-  // k_token_records wrote ([B, L, G] records of REC_FLOATS), or null (each
-  // workgroup builds its tokens itself)
+  // multi-token ridge launches: space for the token records of the row-split
+  // scan ([B, L, G] records of REC_FLOATS), or null (each workgroup builds its
+  // tokens itself)
   const float* rec;
 };
 
@@ -163,8 +159,10 @@ constexpr int tier_packed_of(int j, int T) {
 // INT8 tier is never split between two waves); the other two are the valid
 // cuts that make the largest segment smallest, then the sum of the segments'
 // squares (the lowest cuts on a further tie).  Each
-// segment's readout is one fma chain, and the row's readout their left fold
-// ((s0 + s1) + s2) + s3 on every workgroup shape.  A slot stepped by four
+// segment's readout is one fma chain per tier (ridge: per half, half_pos, the
+// order of its multi-token scan), summed, and the row's readout the segments'
+// left fold ((s0 + s1) + s2) + s3 on every
+// workgroup shape.  A slot stepped by four
 // waves gives wave r segment r; by two waves, wave 0 the segments before the
 // two-wave split and wave 1 the others.
 constexpr bool seg_cut_ok(int n8, int p) { return p <= n8 ? (p % 8 == 0 || p == n8) : (p - n8) % 8 == 0; }
@@ -210,12 +208,33 @@ static_assert(seg_pos(8, 76, 1) == 16 && seg_pos(8, 76, 2) == 40 && seg_pos(8, 7
                   seg_pos(36, 20, 3) == 36 && seg_cuts(36, 20).j == 2 && seg_pos(44, 4, 3) == 44 &&
                   seg_cuts(44, 4).j == 2 && seg_pos(24, 44, 2) == 32 && seg_pos(16, 60, 3) == 56,
               "readout segments");
-// segment of carried coordinate p (the cuts as template-level constants, so
-// that a call with an unrolled loop index folds)
+// Halves of the readout segments: half 2 k is the first part of segment k and
+// half 2 k + 1 the rest, cut at the tier boundary where the segment spans it,
+// else after the larger half of its four-coordinate chunks.  A half lies in
+// one tier (the last may be empty), and the multi-token scan of
+// m2r_rows_kernel.h gives each to a lane.
+constexpr int half_pos(int n8, int n4, int j) {
+  if (j >= 8) return n8 + n4;
+  const int a = seg_pos(n8, n4, j / 2), e = seg_pos(n8, n4, j / 2 + 1);
+  if (j % 2 == 0) return a;
+  return a < n8 && e > n8 ? n8 : a + 4 * ((e - a + 7) / 8);
+}
+// half of carried coordinate p (the cuts as template-level constants, so that
+// a call with an unrolled loop index folds)
 template <int N8, int N4>
-__host__ __device__ __forceinline__ constexpr int seg_of(int p) {
-  constexpr int S1 = seg_pos(N8, N4, 1), S2 = seg_pos(N8, N4, 2), S3 = seg_pos(N8, N4, 3);
-  return p < S1 ? 0 : p < S2 ? 1 : p < S3 ? 2 : 3;
+__host__ __device__ __forceinline__ constexpr int half_of(int p) {
+  constexpr int S1 = half_pos(N8, N4, 1), S2 = half_pos(N8, N4, 2), S3 = half_pos(N8, N4, 3),
+                S4 = half_pos(N8, N4, 4), S5 = half_pos(N8, N4, 5), S6 = half_pos(N8, N4, 6),
+                S7 = half_pos(N8, N4, 7);
+  return p < S4 ? (p < S2 ? (p < S1 ? 0 : 1) : (p < S3 ? 2 : 3)) : (p < S6 ? (p < S5 ? 4 : 5) : (p < S7 ? 6 : 7));
+}
+// readout chain of p: its half, or (MODE other than ridge: one chain per
+// segment and tier) the first half of its segment in its tier
+template <int N8, int N4, int MODE>
+__host__ __device__ __forceinline__ constexpr int chain_of(int p) {
+  const int h = half_of<N8, N4>(p), s = h & ~1;
+  constexpr int HB = half_of<N8, N4>(N8);   // the INT4 tier's first half
+  return MODE == MODE_RIDGE || (s < HB && h >= HB) ? h : s;
 }
 // bit r: wave r of a WPS-wave slot steps INT8 (TIER4 false) or INT4 coordinates
 template <int N8, int N4, int WPS, bool TIER4>
@@ -379,18 +398,6 @@ __device__ __forceinline__ void wave_load_dt(const StepArgs& a, WaveRaw<HPW>& r,
   r.db_lo = db[a.db_f32 ? 2 * h : h];
   r.db_hi = db[a.db_f32 ? 2 * h + 1 : h];
 }
-// x of the wave's rows in each head slot (a record-fed token loop loads
-// only these: dt comes 64 tokens at a time, B and C with the records).
-template <int WPB, int HPW, int WPS = 1>
-__device__ __forceinline__ void wave_load_x(const StepArgs& a, WaveRaw<HPW>& r, int bt, int h0, int pbase, int lane,
-                                            int wave) {
-  const int p = min(pbase + lane, a.P - 1);   // rows past P read row P-1 (never stored)
-#pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const int h = h0 + (WPS > 1 ? wave / WPS : wave * HPW + k);
-    r.xv[k] = a.x[((size_t)bt * a.H + h) * a.P + p];
-  }
-}
 // ALIGNED: B and C are 4-byte aligned, so a lane's pair is one load each.
 template <int WPB, int HPW, bool ALIGNED, int WPS = 1>
 __device__ __forceinline__ void wave_load_rest(const StepArgs& a, WaveRaw<HPW>& r, int bt, int g, int h0,
@@ -408,7 +415,12 @@ __device__ __forceinline__ void wave_load_rest(const StepArgs& a, WaveRaw<HPW>& 
     r.bc[2] = a.Cm[row];
     r.bc[3] = a.Cm[row + 1];
   }
-  wave_load_x<WPB, HPW, WPS>(a, r, bt, h0, pbase, lane, wave);
+  const int p = min(pbase + lane, a.P - 1);   // rows past P read row P-1 (never stored)
+#pragma unroll
+  for (int k = 0; k < HPW; ++k) {
+    const int h = h0 + (WPS > 1 ? wave / WPS : wave * HPW + k);
+    r.xv[k] = a.x[((size_t)bt * a.H + h) * a.P + p];
+  }
 }
 
 // dt activation of head slot `lane` (lanes < HPW; the others compute a copy
@@ -632,35 +644,33 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
 // IEEE product for infinite and NaN scales (where the fused form gives
 // inf - inf).
 //
-// Readout: rs[sg] is set, for each readout segment sg the tier's
-// coordinates reach, to the binary32 chain of prior * w over them (w the
-// readout weights; one segment's chain is live at a time, segments being
-// contiguous runs of chunks).  `bdt4` and `cw4` are the head's B*dt and the
-// readout weights of the carried coordinates, as four-value chunks (BMUL:
-// `bdt4` holds b, and B * dt is formed here with dtk).
+// Readout: rs[hf] is set, for each chain hf (chain_of) in the tier's
+// coordinates, to the binary32 chain of prior * w over them (w the readout
+// weights; one chain is live at a time, chains being contiguous runs of
+// chunks).  `bdt4` and `cw4` are the head's B*dt and the
+// readout weights of the carried coordinates, as four-value chunks.
 //
 // tier_update is the first half (dequantization, readout, update and the
 // maximum of |update|), tier_requant the second (the new scale and codes
 // from the maximum over the whole tier): a tier split between waves runs the
 // halves on its parts with the parts' maxima combined in between.
-template <int N, bool INT8, bool EXACT, int N8, int N4, int P0, bool BMUL = false>
+template <int N, bool INT8, bool EXACT, int N8, int N4, int P0, int MODE>
 __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float decay, float x, const f32x4* bdt4,
-                                             const f32x4* cw4, float (&rs)[4], float (&v)[N], float dtk = 0.f) {
+                                             const f32x4* cw4, float (&rs)[8], float (&v)[N]) {
   constexpr float BIAS = INT8 ? 128.0f : 8.0f;
   static_assert(P0 % 4 == 0 && N % 4 == 0, "whole chunks");
   const float nb = -(1024.0f + BIAS) * sc;
   const f16x2 nbias = {(_Float16)(-(1024.0f + BIAS)), (_Float16)(-(1024.0f + BIAS))};
   const float mz = EXACT ? opaque_neg_zero() : 0.f;
   float amax = 0.f;
-  float racc = 0.f;   // the current segment's readout chain
+  float racc = 0.f;   // the current readout chain
   // the shared operands of chunk i+1 are read while chunk i computes
   constexpr int C0 = P0 / 4;
   f32x4 cb_next = bdt4[C0], cw_next = cw4[C0];
 #pragma unroll
   for (int i0 = 0; i0 < N; i0 += 4) {
     const int ci = C0 + i0 / 4;   // chunk index among the carried coordinates
-    // BMUL: bdt4 holds b, and B * dt is formed here (the same RN(b * dt))
-    const f32x4 cb = BMUL ? cb_next * dtk : cb_next, cw = cw_next;
+    const f32x4 cb = cb_next, cw = cw_next;
     if (i0 + 4 < N) {
       cb_next = bdt4[ci + 1];
       cw_next = cw4[ci + 1];
@@ -672,7 +682,7 @@ __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float 
     asm volatile("" : "+v"(cc));
     const uint32_t h01 = __builtin_amdgcn_perm(0x64646464u, cc, 0x04010400u);
     const uint32_t h23 = __builtin_amdgcn_perm(0x64646464u, cc, 0x04030402u);
-    const int sg = seg_of<N8, N4>(P0 + i0);   // a whole chunk lies in one segment
+    const int hf = chain_of<N8, N4, MODE>(P0 + i0);   // a whole chunk lies in one chain
     float pr[4];
     if constexpr (EXACT) {
       const f16x2 q01 = pk_add_h(__builtin_bit_cast(f16x2, h01), nbias);
@@ -693,26 +703,29 @@ __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float 
     }
     amax = max3_abs(amax, v[i0], v[i0 + 1]);
     amax = max3_abs(amax, v[i0 + 2], v[i0 + 3]);
-    if (i0 + 4 == N || seg_of<N8, N4>(P0 + i0 + 4) != sg) {   // the segment's last chunk in this tier
-      rs[sg] = racc;
+    if (i0 + 4 == N || chain_of<N8, N4, MODE>(P0 + i0 + 4) != hf) {   // the chain's last chunk
+      rs[hf] = racc;
       racc = 0.f;
     }
   }
   // Materialize the readout and the maximum here: otherwise the compiler
   // sinks their chains (and every update behind the maximum) into the
   // requantization, which keeps every prior and LDS operand live at once.
-  constexpr int G0 = seg_of<N8, N4>(P0), G1 = seg_of<N8, N4>(P0 + N - 1);
 #pragma unroll
-  for (int sg = G0; sg <= G1; ++sg) asm volatile("" : "+v"(rs[sg]));
+  for (int i0 = 0; i0 < N; i0 += 4) {
+    const int hf = chain_of<N8, N4, MODE>(P0 + i0);
+    if (i0 + 4 == N || chain_of<N8, N4, MODE>(P0 + i0 + 4) != hf) asm volatile("" : "+v"(rs[hf]));
+  }
   asm volatile("" : "+v"(amax));
   return amax;
 }
 
-// Readout of segment sg: its INT8 tier contribution, then its INT4 one.
-template <int N8, int N4>
-__device__ __forceinline__ float segment_readout(int sg, float c8, float c4) {
-  const bool h8 = seg_pos(N8, N4, sg) < N8, h4 = seg_pos(N8, N4, sg + 1) > N8;
-  return (h8 && h4) ? c8 + c4 : (h8 ? c8 : c4);
+// Readout of segment sg: the sum of its chains.
+template <int N8, int N4, int MODE>
+__device__ __forceinline__ float segment_readout(int sg, const float (&rs)[8]) {
+  const int last = seg_pos(N8, N4, sg + 1) - 1;
+  const bool second = chain_of<N8, N4, MODE>(last) == 2 * sg + 1;
+  return second ? rs[2 * sg] + rs[2 * sg + 1] : rs[2 * sg];
 }
 
 template <int N, bool INT8, int MODE>
@@ -810,7 +823,7 @@ __device__ __forceinline__ float tier_requant(const float (&v)[N], uint32_t* c, 
 // slot's serial chain is about half or a quarter as long; `pacc` and `pmax`
 // pass the waves' readout partial sums and tier maxima (one buffer per token
 // parity).
-template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1, bool REC = false>
+template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1>
 struct StepSmem {
   static constexpr bool PAIR = WPS > 1;
   static_assert(WPS == 1 || ((WPS == 2 || WPS == 4) && HPW == 1 && WPB % WPS == 0),
@@ -821,11 +834,6 @@ struct StepSmem {
   // one-token instances of four or more waves stage their token inputs in
   // LDS by direct transfers (one shared transfer per wave)
   static constexpr bool STAGED = DMA && ONE && WPB >= 4 && NH <= 16;
-  // REC: the record-fed instance (multi-token ridge, several waves per slot,
-  // 16-byte transfers): three record buffers (token t mod 3), and the prior
-  // latent coefficients the last wave of a slot passes to its reading wave
-  // (per token parity)
-  static_assert(!REC || (RIDGE && PAIR && SPLIT && !ONE && DMA), "record-fed instances");
   // slot tile: lo, hi, q4, s8, s4 (and latent) fields of 64 rows, 16 bytes of slack
   static constexpr int TILE = 128 * (N8 / 2) + 64 * (N4 / 2) + 256 + (RIDGE ? 128 : 0) + 16;
   static constexpr int PRED_DW = RIDGE ? F * NZ / 2 : 1;
@@ -836,8 +844,6 @@ struct StepSmem {
   alignas(16) GroupToken<NL> gt[SPLIT && !ONE ? 2 : 1];
   alignas(16) uint32_t pred32[PRED_WORDS];
   alignas(16) std::conditional_t<STAGED, TokenStage, NoStage> stage;
-  alignas(16) float rec[REC ? 3 : 1][REC ? REC_FLOATS : 4];
-  alignas(16) float2 pz[REC ? 2 : 1][REC ? NH : 1][REC ? 64 : 1];
   // WPS > 1 (per token parity): the readout partial sums of waves 0 ..
   // WPS - 2 of a slot, and every wave's maxima of its INT8 and INT4 parts
   alignas(16) float pacc[PAIR ? 2 : 1][PAIR ? NH : 1][PAIR ? WPS : 1][PAIR ? 64 : 1];
@@ -851,9 +857,9 @@ struct StepSmem {
 // The step of one workgroup: block coordinates (bx, by) and batch row b,
 // arguments `a`, LDS `sm`.  k_state_step runs it on its own grid; the
 // multi-layer kernel runs it with arguments read from a table of layers.
-template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1, bool REC = false>
+template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1>
 __device__ __forceinline__ void state_step_body(const StepArgs& a,
-                                                StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS, REC>& sm, int bx,
+                                                StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS>& sm, int bx,
                                                 int by, int b) {
   constexpr bool PAIR = WPS > 1;      // several waves per slot
   constexpr int W8 = N8 / 2;          // bytes per row of lo and of hi
@@ -876,15 +882,9 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
   static_assert(!RIDGE || (F * NZ) % 2 == 0, "predictor staged as dwords");
   static_assert(TILE % 16 == 0, "tiles stay 16-byte aligned");
 
-  using Smem = StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS, REC>;
+  using Smem = StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS>;
   static_assert(Smem::TILE == TILE && Smem::PRED_WORDS == (DMA ? PRED_OPS16 * 256 : PRED_OPS * 64), "LDS layout");
   constexpr bool SPLIT = Smem::SPLIT;
-  // REC, the record-fed token loop (StepArgs::rec): every token's
-  // state-independent values come from its record in LDS.  Wave REC_LOADER
-  // loads record t + 2 while token t steps, and puts record t + 1 in LDS
-  // before token t's maxima barrier, so that the maxima barrier is the only
-  // workgroup barrier of a token (after the first).
-  constexpr int REC_LOADER = 1;
   auto& s_wt = sm.wt;
   auto& s_gt = sm.gt;
   auto& s_pred32 = sm.pred32;
@@ -1087,13 +1087,6 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
   uint32_t basis_w[2] = {0u, 0u};
   uint32_t ls_w = 0u;
   float2 act;
-  // record-fed loop: the loader's copies of records t + 1 and t + 2 (16
-  // bytes per lane), and rec_load(t), this lane's 16 bytes of the record of
-  // token t of the workgroup's batch row and group
-  uint4 rnext = make_uint4(0u, 0u, 0u, 0u), rnext2 = make_uint4(0u, 0u, 0u, 0u);
-  auto rec_load = [&](int t) {
-    return ((const uint4*)(a.rec + ((size_t)(b * L + t) * a.G + g) * REC_FLOATS))[lane];
-  };
   if constexpr (Smem::STAGED) {
     // ---- staged prologue (one token, LDS transfers): the vector inputs of
     // the token and the statics travel by direct transfers into LDS together
@@ -1228,7 +1221,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
     wave_load_dt<WPB, HPW, WPS>(a, raw, b * L, h0, lane, wave);
     const int hl = h0 + head_slot(min(lane, HPW - 1));   // head of slot `lane` (lanes < HPW)
     Ah = a.A[hl];
-    if constexpr (RIDGE && !REC) {   // (a record-fed loop never reads the predictor)
+    if constexpr (RIDGE) {
       const uint8_t* pg = (const uint8_t*)(a.pred + (size_t)g * F * NZ);
       if constexpr (DMA) {   // 16-byte chunks; lanes past the end re-read the last one
         for (int j = wave; j < PRED_OPS16; j += WPB)
@@ -1236,13 +1229,6 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
       } else {
         for (int j = wave; j < PRED_OPS; j += WPB)
           lds_dma_b32(pg + 4 * min(j * 64 + lane, PRED_DW - 1), lds_address(s_pred32 + 64 * j));
-      }
-    }
-    uint4 rec0 = make_uint4(0u, 0u, 0u, 0u);   // REC: record 0, put in LDS once the loads have landed
-    if constexpr (REC) {
-      if (wave == REC_LOADER) {
-        rec0 = rec_load(0);
-        if (L > 1) rnext = rec_load(1);
       }
     }
     wave_load_rest<WPB, HPW, DMA, WPS>(a, raw, b * L, g, h0, pbase, lane, wave);
@@ -1279,9 +1265,6 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
     else {
       for (int k = 0; k < HPW; ++k) slot_copy_in(head_slot(k));
     }
-    if constexpr (REC) {   // record 0, published by the first token's barrier
-      if (wave == REC_LOADER) ((uint4*)sm.rec[0])[lane] = rec0;
-    }
   }
   if (lane < HPW) wt.D[lane] = a.d_f32 ? __builtin_bit_cast(float, d_bits) : h2f((uint16_t)d_bits);
   const int pv0 = perm0 & 127, pv1 = perm1 & 127;   // raw B/C index of internal positions lane, lane + 64
@@ -1306,7 +1289,6 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
   // a wave steps coordinates of a field another wave moves (not so only for
   // two waves split at the tier boundary)
   constexpr bool CROSS = PAIR && !(WPS == 2 && pair_cut(N8, N4) == N8);
-  int rbuf = 0;   // REC: the buffer of token t's record (t mod 3)
   // KEEP (several waves per slot, several tokens): a wave's code words stay
   // in registers from token to token, read from the tile at the first token
   // and written back at the last (no nibble-plane unpacking and repacking
@@ -1318,14 +1300,9 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
   for (int t = 0; t < L; ++t) {
     const int bt = b * L + t;
     const WaveRaw<HPW> cur = raw;
-    if (PAIR && t == ST_TL_TOKEN) M2R_STAMP(ST_TL);
     if (t + 1 < L) {   // prefetch
-      if constexpr (REC) {
-        wave_load_x<WPB, HPW, WPS>(a, raw, bt + 1, h0, pbase, lane, wave);
-      } else {
-        wave_load_dt<WPB, HPW, WPS>(a, raw, bt + 1, h0, lane, wave);
-        wave_load_rest<WPB, HPW, DMA, WPS>(a, raw, bt + 1, g, h0, pbase, lane, wave);
-      }
+      wave_load_dt<WPB, HPW, WPS>(a, raw, bt + 1, h0, lane, wave);
+      wave_load_rest<WPB, HPW, DMA, WPS>(a, raw, bt + 1, g, h0, pbase, lane, wave);
     }
     // readout weights and dead-tier dot products of this token
     const float* cwt;
@@ -1340,22 +1317,8 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
       dot3 = SPLIT ? gt.tree[2] : wt.dots[3];
       dot4 = SPLIT ? gt.tree[3] : wt.dots[4];
     };
-    // REC: record t sits in buffer rbuf (put there before token t - 1's
-    // maxima barrier, or before the first token)
-    const float* rv = sm.rec[REC ? rbuf : 0];
-    if constexpr (REC) {
-      if (t + 2 < L && wave == REC_LOADER) rnext2 = rec_load(t + 2);
-      if (t == 0) __syncthreads();   // record 0 is in LDS
-      cwt = rv + REC_CW;
-      dot1 = rv[REC_TREE] + rv[REC_CW + NL];
-      dot2 = rv[REC_TREE + 1] + rv[REC_CW + NL + 1];
-      dot3 = rv[REC_TREE + 2];
-      dot4 = rv[REC_TREE + 3];
-    } else {
-      build_token();
-    }
+    build_token();
     if (t == 0) M2R_STAMP(ST_BUILD);
-    if (PAIR && t == ST_TL_TOKEN) M2R_STAMP(ST_TL + 1);
 
     for (int k = 0; k < HPW; ++k) {
       // The slot's head index, opaque to the optimizer: every address and
@@ -1386,19 +1349,13 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         // coordinates with the whole tiers' maxima (the same values on every
         // wave, so the same scales and codes as one wave gets) and the last
         // wave steps the latent coefficients and reads the row out. ---------
-        // (REC: from registers and the record: x of the wave's rows, dt and
-        // the decay, the bound flag with the record's flag for b, B * dt
-        // formed in tier_update from the record's b, and sum b.c)
-        const float x = REC ? h2f(cur.xv[0]) : h2f(wt.x[0][lane]);
-        const float decay = REC ? act.y : wt.decay[0];
-        const float dtv = REC ? act.x : wt.dtv[0];
-        const bool bounded = REC ? (rv[REC_BOK] != 0.f && 65504.f * __builtin_fabsf(act.x) < 0x1p100f &&
-                                    __builtin_fabsf(act.y) < 0x1p100f)
-                                 : wt.bounded[0] != 0;
-        const bool base_ok = bounded && __builtin_fabsf(x) <= 65504.f;
-        const f32x4* bdt4 = (const f32x4*)(REC ? rv + REC_B : wt.bdt[0]);
+        const float x = h2f(wt.x[0][lane]);
+        const float decay = wt.decay[0];
+        const float dtv = wt.dtv[0];
+        const bool base_ok = wt.bounded[0] != 0 && __builtin_fabsf(x) <= 65504.f;
+        const f32x4* bdt4 = (const f32x4*)wt.bdt[0];
         const f32x4* cw4 = (const f32x4*)cwt;
-        const float sbc = REC ? rv[REC_SBC] : wt.dots[0];
+        const float sbc = wt.dots[0];
         auto& pacc = sm.pacc[t & 1][hh];
         auto& pmax = sm.pmax[t & 1][hh];
         auto role_body = [&](auto role_c) {
@@ -1417,8 +1374,8 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           constexpr unsigned HAS8 = tier_waves<N8, N4, WPS, false>(), HAS4 = tier_waves<N8, N4, WPS, true>();
           // a tier's maximum is published only when another wave steps part of it
           constexpr bool SHARE8 = (HAS8 & (HAS8 - 1)) != 0, SHARE4 = (HAS4 & (HAS4 - 1)) != 0;
-          // per segment: the tiers' readout chains, then the segment's readout
-          float c8s[4] = {0.f, 0.f, 0.f, 0.f}, c4s[4] = {0.f, 0.f, 0.f, 0.f}, accs[4];
+          // the halves' readout chains, then the segments' readouts
+          float rs[8], accs[4];
           uint32_t c8[M8 > 0 ? (M8 + 3) / 4 : 1], c4[M4 > 0 ? (M4 + 3) / 4 : 1];
           float v8[M8 > 0 ? M8 : 1], v4[M4 > 0 ? M4 : 1];
           float amax8 = 0.f, amax4 = 0.f, s8 = 0.f, s4 = 0.f, z0 = 0.f, z1 = 0.f;
@@ -1427,7 +1384,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           // wave requantized with (every wave of the tier derives the same one)
           // (KEEP: the latent bytes stay in a register where only this last
           // wave reads them, i.e. unless a reading wave reads the tile's)
-          constexpr bool KEEP_LAT = KEEP && (REC || RO == WPS - 1);
+          constexpr bool KEEP_LAT = KEEP && RO == WPS - 1;
           if constexpr (M8 > 0) {
             if (KEEP && t > 0) {
 #pragma unroll
@@ -1446,22 +1403,17 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
             }
             fin8 = __builtin_fabsf(s8) <= 65504.f;
             if (__builtin_amdgcn_ballot_w64(!fin8) == 0)
-              amax8 = tier_update<M8, true, false, N8, N4, A8, REC>(c8, s8, decay, x, bdt4, cw4, c8s, v8, dtv);
+              amax8 = tier_update<M8, true, false, N8, N4, A8, MODE>(c8, s8, decay, x, bdt4, cw4, rs, v8);
             else
-              amax8 = tier_update<M8, true, true, N8, N4, A8, REC>(c8, s8, decay, x, bdt4, cw4, c8s, v8, dtv);
+              amax8 = tier_update<M8, true, true, N8, N4, A8, MODE>(c8, s8, decay, x, bdt4, cw4, rs, v8);
             if constexpr (SHARE8) pmax[0][R][lane] = amax8;
           }
-          // the latent coefficients, read with the rows (REC: by the last
-          // wave only, which passes them to the reading wave through pz: the
-          // tile's latent bytes of token t are rewritten after the barrier
-          // without another barrier before token t + 1)
-          constexpr bool PASS_Z = REC && READS_OUT != LAST;
-          if constexpr ((LAST || (READS_OUT && !PASS_Z)) && RIDGE) {
+          // the latent coefficients, read with the rows
+          if constexpr ((LAST || READS_OUT) && RIDGE) {
             const uint32_t lat = (KEEP_LAT && LAST && t > 0) ? keep_lat : (uint32_t)t16[O_LAT / 2 + lane];
             z0 = e4m3_byte_to_f32<0>(lat) * ls0;
             z1 = e4m3_byte_to_f32<1>(lat) * ls1;
             if (PLACEHOLDERS && !valid) z0 = z1 = 0.f;
-            if constexpr (PASS_Z && LAST) sm.pz[t & 1][hh][lane] = make_float2(z0, z1);
           }
           if constexpr (M4 > 0) {
             if (KEEP && t > 0) {
@@ -1480,9 +1432,9 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
             }
             fin4 = __builtin_fabsf(s4) <= 65504.f;
             if (__builtin_amdgcn_ballot_w64(!fin4) == 0)
-              amax4 = tier_update<M4, false, false, N8, N4, N8 + A4, REC>(c4, s4, decay, x, bdt4, cw4, c4s, v4, dtv);
+              amax4 = tier_update<M4, false, false, N8, N4, N8 + A4, MODE>(c4, s4, decay, x, bdt4, cw4, rs, v4);
             else
-              amax4 = tier_update<M4, false, true, N8, N4, N8 + A4, REC>(c4, s4, decay, x, bdt4, cw4, c4s, v4, dtv);
+              amax4 = tier_update<M4, false, true, N8, N4, N8 + A4, MODE>(c4, s4, decay, x, bdt4, cw4, rs, v4);
             if constexpr (SHARE4) pmax[1][R][lane] = amax4;
           }
           uint32_t qz = 0;
@@ -1497,25 +1449,15 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           // the left fold of the readout segments: the other waves publish
           // the fold of their segments, the reading wave folds them in order
 #pragma unroll
-          for (int sg = G0; sg < G1; ++sg) accs[sg] = segment_readout<N8, N4>(sg, c8s[sg], c4s[sg]);
+          for (int sg = G0; sg < G1; ++sg) accs[sg] = segment_readout<N8, N4, MODE>(sg, rs);
           float part = accs[G0];
 #pragma unroll
           for (int sg = G0 + 1; sg < G1; ++sg) part = part + accs[sg];
           if constexpr (!READS_OUT) pacc[R][lane] = part;
-          if constexpr (REC) {   // record t + 1 into the buffer token t - 2 used (every wave is past it)
-            if (wave == REC_LOADER && t + 1 < L) ((uint4*)sm.rec[rbuf == 2 ? 0 : rbuf + 1])[lane] = rnext;
-          }
           if (t == 0) M2R_STAMP(ST_SLOT + 1);
-          if (t == ST_TL_TOKEN) M2R_STAMP(ST_TL + 2);
           __syncthreads();   // readout partials and tier maxima are published
           if (t == 0) M2R_STAMP(ST_SLOT + 2);
-          if (t == ST_TL_TOKEN) M2R_STAMP(ST_TL + 3);
           if constexpr (READS_OUT) {
-            if constexpr (PASS_Z && RIDGE) {
-              const float2 zz = sm.pz[t & 1][hh][lane];
-              z0 = zz.x;
-              z1 = zz.y;
-            }
             float acc = RO == 0 ? part : pacc[0][lane];
 #pragma unroll
             for (int r = 1; r < WPS; ++r) {
@@ -1590,10 +1532,10 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         const bool base_ok = wt.bounded[k] != 0 && __builtin_fabsf(x) <= 65504.f;
         const f32x4* bdt4 = (const f32x4*)wt.bdt[k];
         const f32x4* cw4 = (const f32x4*)cwt;
-        // the readout per readout segment: each tier's contribution, then the
-        // segment's sum, folded after both tiers (the order of the multi-wave
-        // slots, whose segments run on different waves)
-        float c8s[4] = {0.f, 0.f, 0.f, 0.f}, c4s[4] = {0.f, 0.f, 0.f, 0.f};
+        // the readout per half of the readout segments, folded after both
+        // tiers (the order of the multi-wave slots, whose segments run on
+        // different waves)
+        float rs[8];
 
         // ---- INT8 tier: unpack (byte k of c8[i] is q8 + 128 of internal
         // coordinate 4i+k), update with readout accumulation, requantize and
@@ -1621,10 +1563,10 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           {
             float v8[N8];
             if (__builtin_amdgcn_ballot_w64(!fin8) == 0) {
-              const float m8 = tier_update<N8, true, false, N8, N4, 0>(c8, sc8, decay, x, bdt4, cw4, c8s, v8);
+              const float m8 = tier_update<N8, true, false, N8, N4, 0, MODE>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
               sc8 = tier_requant<N8, true, MODE>(v8, c8, m8, base_ok);
             } else {
-              const float m8 = tier_update<N8, true, true, N8, N4, 0>(c8, sc8, decay, x, bdt4, cw4, c8s, v8);
+              const float m8 = tier_update<N8, true, true, N8, N4, 0, MODE>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
               sc8 = tier_requant<N8, true, MODE>(v8, c8, m8, base_ok && fin8);
             }
           }
@@ -1672,10 +1614,10 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         {
           float v4[N4];
           if (__builtin_amdgcn_ballot_w64(!fin4) == 0) {
-            const float m4 = tier_update<N4, false, false, N8, N4, N8>(c4, sc4, decay, x, bdt4, cw4, c4s, v4);
+            const float m4 = tier_update<N4, false, false, N8, N4, N8, MODE>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
             sc4 = tier_requant<N4, false, MODE>(v4, c4, m4, base_ok);
           } else {
-            const float m4 = tier_update<N4, false, true, N8, N4, N8>(c4, sc4, decay, x, bdt4, cw4, c4s, v4);
+            const float m4 = tier_update<N4, false, true, N8, N4, N8, MODE>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
             sc4 = tier_requant<N4, false, MODE>(v4, c4, m4, base_ok && fin4);
           }
         }
@@ -1685,7 +1627,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         __builtin_amdgcn_sched_barrier(0);
         float accs[4];
 #pragma unroll
-        for (int sg = 0; sg < 4; ++sg) accs[sg] = segment_readout<N8, N4>(sg, c8s[sg], c4s[sg]);
+        for (int sg = 0; sg < 4; ++sg) accs[sg] = segment_readout<N8, N4, MODE>(sg, rs);
         const float acc = ((accs[0] + accs[1]) + accs[2]) + accs[3];   // the readout segments' left fold
         // readout: sum_i u_i c_i + corrections = decay * (sum_i prior_i (c_i +
         // corr_i) + latent terms) + x * (dt * sum_all b c + D)
@@ -1719,13 +1661,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
       }
       wave_sync();
       if (t == 0 && k < 4) M2R_STAMP(ST_SLOT + 4 * k + 3);
-      if (PAIR && t == ST_TL_TOKEN) M2R_STAMP(ST_TL + 4);
     }
-    if constexpr (REC) {
-      rbuf = rbuf == 2 ? 0 : rbuf + 1;
-      if (wave == REC_LOADER) rnext = rnext2;
-    }
-    if (PAIR && t == ST_TL_TOKEN) M2R_STAMP(ST_TL + 5);
     if (t == L - 1) {
       // ... and the moving wave writes back every wave's last values
       if constexpr (CROSS) __syncthreads();
@@ -1749,16 +1685,16 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
 #endif
 }
 
-template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1, bool REC = false>
+template <int N8, int N4, int NZ, int MODE, int WPB, int HPW, bool DMA, bool ONE, int WPS = 1>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(WPB == 8 && WPS == 1 ? 4 : 2, 8)))
 void k_state_step(StepArgs a) {
-  __shared__ StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS, REC> sm;
-  state_step_body<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS, REC>(a, sm, blockIdx.x, blockIdx.y, blockIdx.z);
+  __shared__ StepSmem<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS> sm;
+  state_step_body<N8, N4, NZ, MODE, WPB, HPW, DMA, ONE, WPS>(a, sm, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // ---------------------------------------------------------------------------
-// Token records of a multi-token ridge launch (the record-fed token loop of
-// k_state_step): one four-wave workgroup per (REC_TOKENS tokens, group,
+// Token records of a multi-token ridge launch (read by the row-split scan,
+// m2r_rows_kernel.h): one four-wave workgroup per (REC_TOKENS tokens, group,
 // batch row) runs the split token build of every token (wave_token_build with
 // four waves: the same gathers, sums, ridge correction and dead-tier trees,
 // so the same bits) and wave 0 stores the state-independent values as the

@@ -57,12 +57,20 @@ def launch_packed(kind, x, dt, A, B, C, D, dt_bias, perm, tensors, *, n8, n4, nz
         common = (p(x), p(dt), p(A), p(B), p(C), p(D), d_f32, p(dt_bias), db_f32, p(perm))
         geo = (batch, length, heads, dim, groups)
         if kind == "ridge":
-            # multi-token calls on the small-batch shapes (at most 1024 64-row
-            # slots) take a token-record workspace (results identical without)
+            # a token-record workspace (results identical without) where the
+            # scan that reads the records beats building each token in the
+            # step kernel; us per call, built / records, at batch 1, 8 and 64
+            # (24/44/60): 16 tokens 30.8 / 28.2, 46.2 / 48.4, 263.8 / 227.9;
+            # 8 tokens 17.9 / 23.8, 26.2 / 36.9, 145.3 / 146.2; wide rows over
+            # many slots 8/76/44 at batch 16, 64 tokens 286 / 273.  Bounded to
+            # 1 GiB beyond 1024 64-row slots.
             ws, ws_bytes = None, 0
-            if length > 1 and batch * heads * -(-dim // 64) <= 1024:
-                ws_bytes = int(_native.lib().m2r_ridge_records_bytes(batch, length, groups))
-                ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
+            slots = batch * heads * -(-dim // 64)
+            if length >= (16 if slots <= 384 else 24 if slots <= 1024 or n8 + n4 <= 72 else 64):
+                need = int(_native.lib().m2r_ridge_records_bytes(batch, length, groups))
+                if need <= 1 << 30 or slots <= 1024:
+                    ws_bytes = need
+                    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
             _native.call("m2r_state_step_ridge_ws", *common, p(basis.contiguous()), p(lscale.contiguous()),
                          p(pred.contiguous()), p(tensors["lo"]), p(tensors["hi"]), p(tensors["q4"]),
                          p(tensors["latent"]), p(tensors["s8"]), p(tensors["s4"]), p(y), *geo, n8, n4, nz,

@@ -650,6 +650,54 @@ def test_packed_rows_non_finite_scales(oracle, device):
              special_scales=NONFINITE_SCALES)
 
 
+# (batch, L, H, P, G) of the multi-token scans with rows on 8, 8, 8, 4, 2 and
+# 1 or 4 lanes (by the 64-row slots; more than 72 carried coordinates: 4):
+# heads per group 1, 6, 16 and 2, one, two and four heads per workgroup,
+# waves with no, some and all rows valid, token counts around the blocks of 16
+# and the dt batches of 64
+ROWS_CASES = [(1, 17, 8, 80, 8), (1, 65, 12, 48, 2), (3, 24, 128, 16, 8), (5, 33, 128, 32, 8), (8, 47, 128, 48, 8),
+              (13, 64, 128, 16, 8), (13, 66, 128, 80, 64)]
+
+
+@pytest.mark.parametrize("case", range(len(ROWS_CASES)))
+@pytest.mark.parametrize("codec", ["ridge", "tier", "legacy", "permutation", "equalizer"])
+def test_rows_scan_lanes_and_edges(oracle, device, case, codec):
+    batch, L, H, P, G = ROWS_CASES[case]
+    if codec == "ridge":   # (P % 16 == 0)
+        for layout in (RIDGE_LAYOUTS[case % 7], RIDGE_LAYOUTS[(case + 3) % 7]):
+            run_ridge(oracle, device, layout, batch, L, H, P, G, 3100 + case, d_f32=case % 2 == 1,
+                      db_f32=case % 3 == 1, dt_bias_zero=False)
+    elif codec in ("tier", "legacy"):
+        for layout in (TIER_LAYOUTS[case % 7], TIER_LAYOUTS[(case + 3) % 7]) if codec == "tier" else ("16_64_48",):
+            run_tier(oracle, device, codec, layout, batch, L, H, P - 8, G, 3200 + case, d_f32=case % 2 == 1,
+                     db_f32=case % 3 == 1, dt_bias_zero=False)
+    else:
+        run_dense3(oracle, device, codec, batch, L, H, P - 8, G, 3300 + case)
+
+
+@pytest.mark.parametrize("batch,L", [(1, 24), (5, 24), (8, 24), (13, 64)])
+def test_rows_scan_unusual_states(oracle, device, batch, L):
+    """Zero states, binary16-subnormal stored scales and non-finite stored
+    scales on 8, 4, 2 and 1 or 4 lanes per row."""
+    H, P, G = 128, 16, 8
+    for i, layout in enumerate(("24_48_56", "44_8_76", "8_80_40")):
+        run_ridge(oracle, device, layout, batch, L, H, P, G, 3400 + i, random_state=False)
+        run_ridge(oracle, device, layout, batch, L, H, P, G, 3410 + i, x_scale=3e-7, scale_mu=-17.0)
+        # An infinite scale reads out as (c + correction) inf here and as
+        # c inf + correction inf in the oracle: NaN on one side only where
+        # every coordinate of the tier gives one sign, as four coordinates
+        # (44_8_76's INT4 tier) do in one row of eight, and 32 in none.
+        run_ridge(oracle, device, "32_32_64" if layout == "44_8_76" else layout, batch, L, H, P, G, 3420 + i,
+                  special_scales=NONFINITE_SCALES)
+        run_tier(oracle, device, "tier", layout, batch, L, H, P, G, 3430 + i, special_scales=NONFINITE_SCALES)
+    run_tier(oracle, device, "legacy", "16_64_48", batch, L, H, P, G, 3440, random_state=False)
+    run_tier(oracle, device, "legacy", "16_64_48", batch, L, H, P, G, 3441, special_scales=NONFINITE_SCALES)
+    run_dense3(oracle, device, "permutation", batch, L, H, P, G, 3450, random_state=False)
+    run_dense3(oracle, device, "permutation", batch, L, H, P, G, 3451, x_scale=1e-9, scale_mu=-24.0)
+    run_dense3(oracle, device, "equalizer", batch, L, H, P, G, 3452, special_scales=NONFINITE_SCALES,
+               nonfinite_y=True)
+
+
 def run_s16(oracle, device, batch, L, H, P, G, seed, collect):
     from mamba2_recall import state_codec
     rng = np.random.default_rng(seed)
