@@ -174,6 +174,49 @@ def test_g64_random_bit_exact(oracle, device, rows, cols):
     assert int((got != want).sum()) == 0
 
 
+@pytest.mark.parametrize("group", [16, 64])
+@pytest.mark.parametrize("rows,cols", [(3, 8), (5, 9), (2, 15), (7, 17), (67, 31), (1000, 33), (129, 63), (5, 65),
+                                       (3, 2730), (3, 2731), (9, 4100), (2, 8191), (3, 8193), (1, 20001), (4, 7)])
+def test_ragged_widths_bit_exact(oracle, device, group, rows, cols):
+    """Widths that are no multiple of the group: rows and groups that end
+    anywhere in an eight-weight vector, a partial last vector, widths on both
+    sides of a workgroup's 8192 weights, and one below eight columns."""
+    if cols % group == 0:
+        return
+    rng = np.random.default_rng(rows * 31 + cols + group)
+    groups = (cols + group - 1) // group
+    codes = rng.integers(0, 16, size=(rows, groups * group)).astype(np.uint8)
+    codes[:, cols:] = 0
+    packed = (codes[:, 0::2] | (codes[:, 1::2] << 4)).astype(np.uint8)
+    s = np.exp(rng.normal(-3.0, 0.5, size=(rows, groups))).astype(np.float32)
+    g = np.float32(s.max() / 448.0)
+    if group == 16:
+        sc = torch.from_numpy(np.clip(s / g, 0, 448)).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+    else:
+        sc, g = s.astype(np.float16).view(np.uint16), None
+    print(f"[fp4 ragged] group={group} rows={rows} cols={cols}", flush=True)
+    want, err = oracle.fp4_decode(group, packed, sc, 1.0 if g is None else g, rows, cols)
+    assert err == 0
+    got = decode_dev(packed, sc, g, rows, cols, device, group=group).cpu().numpy().view(np.uint16)
+    assert int((got != want).sum()) == 0
+    if rows > 2:   # the error bits, in the middle and at the ends
+        for r, c in ((0, cols - 1), (rows // 2, 0), (rows - 1, cols // 2), (rows - 1, cols - 1)):
+            bad = sc.copy()
+            bad[r, c // group] = 0
+            pk = packed.copy()
+            pk[r, c // 2] = 0x11 & (0x0F if cols % 2 and c == cols - 1 else 0xFF)
+            with pytest.raises(ValueError, match="Nonzero code in a zero-scale group"):
+                decode_dev(pk, bad, g, rows, cols, device, group=group)
+            bad[r, c // group] = 0x7F if group == 16 else 0x7E00
+            with pytest.raises(ValueError, match="Invalid stored scale"):
+                decode_dev(packed, bad, g, rows, cols, device, group=group)
+        for r, c in ((0, cols), (rows - 1, groups * group - 1), (rows // 2, cols)):
+            pk = packed.copy()
+            pk[r, c // 2] |= 0x10 if c % 2 else 0x01
+            with pytest.raises(ValueError, match="Nonzero final-group padding"):
+                decode_dev(pk, sc, g, rows, cols, device, group=group)
+
+
 def test_decode_errors_follow_reference_order(device):
     rng = np.random.default_rng(5)
     rows, cols = 4, 64
