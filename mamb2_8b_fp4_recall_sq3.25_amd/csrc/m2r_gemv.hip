@@ -27,7 +27,8 @@
 // order.  A wave sum per chunk, then the chunks' partial sums in a fixed
 // order through LDS, finish each output.  One activation row (the batch-1
 // decode) takes k_fp4_gemv_rows instead where it fills the chip in one
-// resident round: whole rows per wave, no barrier per row, the same sums.
+// resident round: whole rows per wave, no barrier per row, the same sums.  Four
+// rows take k_fp4_gemv_tiles (matrix cores).
 #include "m2r_device.h"
 #include "m2r_abi_util.h"
 #include "m2r_tile.h"
@@ -257,6 +258,131 @@ __global__ __launch_bounds__(64 * WPB) void k_fp4_gemv_rows(const uint8_t* __res
   }
 }
 
+// Four activation rows: with a dot product per row and weight pair the vector
+// units have 3.4 instructions a weight, twice the 1.6 that form it, and the
+// sums of four rows; the matrix cores take the products and sums off them.  A
+// workgroup of NW waves takes tiles of 16 matrix rows, wave w the w-th part of
+// K, as v_mfma_f32_16x16x32_f16 with the 16 rows of weights (A) against the
+// four activation rows (B; the other 12 columns repeat the last one, unused).
+// A lane's eight k of an A operand are one code word, in the order in which
+// the permutes leave them; the B fragments stay in registers for every tile,
+// reordered once to match.  One workgroup per CU, AHEAD tiles of loads in
+// flight; the waves' partial sums of up to eight tiles wait in LDS for one
+// barrier.  us per launch, dot products / tiles: [18560, 4096] 23.7 / 15.8,
+// [4096, 8192] 16.7 / 11.4, [18560, 2048] 16.9 / 8.7, [4096, 4096] 12.9 / 6.5,
+// [64000, 4096] 61.1 / 39.5.  (One and two rows keep the dot products: one
+// row 14.1 / 15.7 and 8.2 / 10.9 on the first two, and two sum as one does.)
+// More tiles ahead or waves per workgroup, and conflict-free table reads,
+// measure the same: what bounds it is issuing the 14 vector instructions per
+// code word, with the matrix instructions between them.
+constexpr int GEMV_TILES = 8;   // tiles whose partial sums wait in LDS for one barrier
+typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
+
+template <int KCH, int NW, int AHEAD>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 16 ? 4 : 2, 8)))
+void k_fp4_gemv_tiles(const uint8_t* __restrict__ codes, const uint8_t* __restrict__ scales,
+                      const float* __restrict__ gscale, const uint16_t* __restrict__ u, int64_t u_stride,
+                      uint16_t* __restrict__ y, int64_t y_stride, int N) {
+  constexpr int M = 4;
+  constexpr int K = KCH * 2048, KW = K / NW, I = KW / 128;
+  __shared__ __align__(16) uint32_t s_tab[128][4];
+  __shared__ __align__(16) float s_part[GEMV_TILES][NW][16][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c16 = lane & 15, g = lane >> 4;
+  const int k0 = wave * KW + 32 * g;   // the lane's first k; its pieces of 32 lie 128 apart
+  const int tiles = (N + 15) / 16, stride = gridDim.x;
+  u32x4 cv[AHEAD][I];
+  uint32_t sb[AHEAD][I];
+  auto load_tile = [&](int tile, u32x4 (&c)[I], uint32_t (&s)[I]) {
+    const int row = min(16 * tile + c16, N - 1);   // rows past N re-read row N-1 (never stored)
+    const uint8_t* pc = codes + (size_t)row * (K / 2) + k0 / 2;
+    const uint8_t* ps = scales + (size_t)row * (K / 16) + k0 / 16;
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      c[i] = *(const u32x4*)(pc + 64 * i);
+      s[i] = *(const uint16_t*)(ps + 8 * i);
+    }
+  };
+  // the activations first (cache hits, shared by every workgroup), so that
+  // waiting for them does not wait for the tiles.  Columns past M repeat the
+  // last row (their products are never stored).
+  u32x4 uv[I][4];
+  const uint16_t* pu = u + min(c16, M - 1) * u_stride + k0;
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) uv[i][j] = *(const u32x4*)(pu + 128 * i + 8 * j);
+#pragma unroll
+  for (int p = 0; p < AHEAD; ++p)
+    if ((int)blockIdx.x + p * stride < tiles) load_tile(blockIdx.x + p * stride, cv[p], sb[p]);
+  const float gl = *gscale;
+  for (int e = threadIdx.x; e < 128 * 8; e += 64 * NW) {
+    const int blk = e >> 3, i = e & 7;
+    const float lev2 = (float)((i < 4) ? i : (i == 4 ? 4 : (i == 5 ? 6 : (i == 6 ? 8 : 12))));
+    const float hb = e4m3_byte_to_f32<0>((uint32_t)blk) * 0.5f;
+    const uint16_t h = f2h((lev2 * hb) * gl);
+    uint8_t* row = (uint8_t*)s_tab[blk];
+    row[i] = (uint8_t)(h & 0xFFu);
+    row[8 + i] = (uint8_t)(h >> 8);
+  }
+  // pairs in the weights' order: (u0,u2), (u4,u6), (u1,u3), (u5,u7)
+  gh8 bf[I][4];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32x4 v = uv[i][j];
+      const u32x4 r = {__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
+                       __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u)};
+      bf[i][j] = __builtin_bit_cast(gh8, r);
+    }
+  __syncthreads();   // the table is complete
+  for (int first = blockIdx.x; first < tiles; first += GEMV_TILES * stride) {
+    for (int t0 = 0; t0 < GEMV_TILES && first + t0 * stride < tiles; t0 += AHEAD) {
+#pragma unroll
+      for (int p = 0; p < AHEAD; ++p) {
+        const int t = t0 + p, tile = first + t * stride;
+        if (tile < tiles) {
+          f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+          for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const u32x4 tv = *(const u32x4*)s_tab[(sb[p][i] >> (8 * (j >> 1))) & 0x7Fu];
+              const uint32_t cw = cv[p][i][j];
+              const uint32_t even = cw & 0x07070707u, odd = (cw >> 4) & 0x07070707u;
+              const uint32_t le = __builtin_amdgcn_perm(tv.y, tv.x, even), lo = __builtin_amdgcn_perm(tv.y, tv.x, odd);
+              const uint32_t he = __builtin_amdgcn_perm(tv.w, tv.z, even) | ((cw & 0x08080808u) << 4);
+              const uint32_t ho = __builtin_amdgcn_perm(tv.w, tv.z, odd) | (cw & 0x80808080u);
+              const u32x4 w = {__builtin_amdgcn_perm(he, le, 0x05010400u), __builtin_amdgcn_perm(he, le, 0x07030602u),
+                               __builtin_amdgcn_perm(ho, lo, 0x05010400u), __builtin_amdgcn_perm(ho, lo, 0x07030602u)};
+              acc[j & 1] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gh8, w), bf[i][j], acc[j & 1], 0, 0, 0);
+            }
+          if (tile + AHEAD * stride < tiles) load_tile(tile + AHEAD * stride, cv[p], sb[p]);
+          const f32x4 sum = acc[0] + acc[1];   // rows 4 g .. 4 g + 3 of column c16
+          if (c16 < 4) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s_part[t][wave][4 * g + q][c16] = sum[q];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // output (tile t, row m of y, weight row): the waves' sums in order
+    for (int e = threadIdx.x; e < GEMV_TILES * 64; e += 64 * NW) {
+      const int t = e >> 6, m = (e >> 4) & 3, row = e & 15, n = 16 * (first + t * stride) + row;
+      if (m < M && n < N) {
+        float s = s_part[t][0][row][m];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) s = s + s_part[t][w][row][m];
+        y[m * y_stride + n] = f2h(s);
+      }
+    }
+    __syncthreads();
+  }
+}
+
 }  // namespace m2r
 
 using namespace m2r;
@@ -325,6 +451,22 @@ extern "C" int m2r_fp4_gemv_g16(const uint8_t* packed, const uint8_t* e4m3_scale
   if ((((uintptr_t)packed | (uintptr_t)u) & 15) || (u_stride % 8) || ((uintptr_t)e4m3_scales & 1))
     return m2r_fail("fp4 gemv: codes and activation rows must be 16-byte aligned, scales 2-byte aligned");
   const int kch = (int)(K / 2048);
+  if (M == 4) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      return m2r_fail("fp4 gemv: device query failed");
+    const dim3 grid((unsigned)std::min<int64_t>((N + 15) / 16, cus));
+#define M2R_TILES(KK, NW, AHEAD)                                                                              \
+    if (kch == KK) {                                                                                          \
+      hipLaunchKernelGGL((k_fp4_gemv_tiles<KK, NW, AHEAD>), grid, dim3(64 * NW), 0, stream, packed,           \
+                         e4m3_scales, global_scale, (const uint16_t*)u, u_stride, (uint16_t*)y, y_stride,     \
+                         (int)N);                                                                             \
+      return m2r_check(hipGetLastError(), "fp4 gemv launch");                                                 \
+    }
+    M2R_TILES(1, 8, 2) M2R_TILES(2, 8, 2) M2R_TILES(4, 16, 1)
+#undef M2R_TILES
+  }
   if (M == 1) {
     if (int e = launch_rows(kch, packed, e4m3_scales, global_scale, (const uint16_t*)u, (uint16_t*)y, N, stream))
       return e > 0 ? m2r_check(hipGetLastError(), "fp4 gemv launch") : 1;
@@ -341,7 +483,6 @@ extern "C" int m2r_fp4_gemv_g16(const uint8_t* packed, const uint8_t* e4m3_scale
   }
   M2R_GEMV(1, 1) M2R_GEMV(1, 2) M2R_GEMV(1, 4)
   M2R_GEMV(2, 1) M2R_GEMV(2, 2) M2R_GEMV(2, 4)
-  M2R_GEMV(4, 1) M2R_GEMV(4, 2) M2R_GEMV(4, 4)
 #undef M2R_GEMV
   return m2r_fail("fp4 gemv: supported are M in {1, 2, 4} rows of u and K in {2048, 4096, 8192}");
 }

@@ -275,6 +275,34 @@ def test_fp4_gemv_matches_decoded_weights(device, M, N, K):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("N,K,tiny", [(1, 4096, 1.0), (16, 8192, 1.0), (17, 2048, 1.0), (4111, 4096, 1.0),
+                                      (40003, 2048, 1.0), (5000, 8192, 2.0 ** -16)])
+def test_fp4_gemv_four_rows_tiles(device, N, K, tiny):
+    """The matrix-core GEMV (four activation rows) around its 16-row tiles and
+    its batches of eight tiles per workgroup (N > 32,768), and with weights
+    down to binary16 subnormals, against float64 within the bound of the test
+    above: products of binary16 values are exact in binary32."""
+    from mamba2_recall import fp4
+    gen = torch.Generator(device=device).manual_seed(N + K)
+    print(f"[fp4 gemv tiles] N={N} K={K} tiny={tiny}", flush=True)
+    codes = torch.randint(0, 256, (N, K // 2), generator=gen, device=device, dtype=torch.uint8)
+    s = torch.exp(torch.randn((N, K // 16), generator=gen, device=device) * 0.5 - 3.0)
+    g = (s.max() / 448.0).float().reshape(1)
+    sb = (s / g).clamp(0, 448).to(torch.float8_e4m3fn).view(torch.uint8)
+    sb = torch.where(sb == 0, torch.ones_like(sb), sb)
+    g = g * tiny
+    w = fp4.decode_packet(dict(format="fp4_g16_e4m3", shape=[N, K], group_size=16, packed=codes,
+                               scales=sb.view(torch.float8_e4m3fn), global_scale=g.reshape(())))
+    if tiny < 1:
+        assert float((w.abs().float() < 2.0 ** -14).float().mean()) > 0.5
+    wide = torch.randn((4, K + 8), generator=gen, device=device).half()
+    for u in (wide[:, :K].contiguous(), wide[:, :K]):   # the second with a row stride of its own
+        y = fp4.gemv_g16(codes, sb, g, u)
+        ref = u.double() @ w.double().T
+        bound = (ref.abs() * 2.0 ** -11 + (u.double().abs() @ w.double().abs().T) * K * 2.0 ** -22 + 2.0 ** -24)
+        assert bool(((y.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("N,K", [(18560, 4096), (4640, 4096), (4096, 8192), (2048, 8192), (100, 2048)])
 def test_fp4_gemv_one_row_same_bits_as_two_rows(device, N, K):
     """One activation row runs the whole-row kernel where it fills the chip in
