@@ -306,6 +306,26 @@ int m2r_causal_conv_update(void* window, int64_t ws_b, int64_t ws_c, int64_t ws_
                            int width, int silu, hipStream_t stream);
 
 /*
+ * Causal depthwise convolution and SiLU of `tokens` tokens (the prefill form
+ * of the update above), writing the three channel ranges the scan takes as
+ * separate contiguous tensors.  The binary64 sum is rounded through
+ * binary32 to binary16, the bias added in binary16, then the SiLU.  Replaces the PyTorch branch of
+ * mamba2_recall/state_quant.py:305-317.
+ *   window f16 [B, C, width] by element strides ws_b, ws_t (channel stride
+ *   1): with history != 0 its last three inputs precede the first token, else
+ *   nothing does; on return it holds the last four inputs, zeros before them.
+ *   value f16 [B, tokens, C] with strides vs_b, vs_l (channel stride 1);
+ *   weight f16 [C, width] contiguous; bias f16 [C] or NULL; x, bm, cm f16
+ *   [B, tokens, n_x | n_b | n_c] contiguous, C = n_x + n_b + n_c.
+ * width must be 4; channel counts and strides multiples of 4, operands
+ * 8-byte aligned; the window and value must not overlap an output.
+ */
+int m2r_causal_conv_tokens(void* window, int64_t ws_b, int64_t ws_t, int history, const void* value, int64_t vs_b,
+                           int64_t vs_l, const void* weight, const void* bias, void* x, void* bm, void* cm,
+                           int64_t n_x, int64_t n_b, int64_t n_c, int64_t batch, int64_t tokens, int width,
+                           hipStream_t stream);
+
+/*
  * Gated RMS norm of the Mamba-2 mixer, norm_before_gate = False: per group of
  * group_size channels of each row, v = y * (z * sigmoid(z)) in binary32,
  * out = half((v / sqrt(mean(v^2) + eps)) * weight).  Replaces the gated norm

@@ -62,6 +62,148 @@ extern "C" int m2r_causal_conv_update(void* window, int64_t ws_b, int64_t ws_c, 
 }
 
 // ---------------------------------------------------------------------------
+// Causal depthwise convolution of several tokens, the prefill form of the
+// update above (the PyTorch branch of mamba2_recall/state_quant.py:305-317):
+//   s   = half(float(sum_k x[t - 3 + k] * w[k])) (binary64 sum, as the library rounds it)
+//   s   = half(s + bias)                       (when a bias is given)
+//   out = half(s / (1 + exp(-s)))              (silu in binary32)
+// x before the first token is the cached window's last three inputs when the
+// request has a history; without one those taps are left out (not multiplied
+// by zero).  The window then holds the last four inputs.
+//
+// Bound: about 45 vector instructions per output (four binary64 products, the
+// roundings, exp and divide) next to two bytes read and two written.  As
+// library calls this was a transposing copy, a convolution with strided
+// stores, a bias pass, a SiLU pass and three copies that split the channels:
+// 1024 tokens of 10240 channels took about 160 us of a mixer call, and take
+// 18 us here (42 MB, 8 us at the rate of a copy).  A thread keeps the window
+// of four neighbouring channels in registers over kConvSeg tokens, reads the
+// projection's rows in place and writes x, B and C as the contiguous tensors
+// the scan reads.  Eight channels per thread need 167 registers, and 2.5
+// waves per SIMD took 22 us.
+namespace m2r {
+
+constexpr int kConvSeg = 8;   // tokens per thread: 3 inputs read again per 8, and five waves per SIMD at that size
+
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+
+struct ConvArgs {
+  uint16_t* window;
+  int64_t ws_b, ws_t;
+  const uint16_t* value;
+  int64_t vs_b, vs_l;
+  const uint16_t *weight, *bias;
+  uint16_t* out[3];
+  int64_t n[3];   // channels of each output
+  int64_t batch, tokens, segs;
+  int history;
+};
+
+__global__ __launch_bounds__(256) void k_conv_tokens(ConvArgs a) {
+  const int64_t chunks = (a.n[0] + a.n[1] + a.n[2]) / 4;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= chunks * a.segs * a.batch) return;
+  const int64_t chunk = i % chunks;
+  i /= chunks;
+  const int64_t seg = i % a.segs, b = i / a.segs;
+  int64_t c = chunk * 4;
+  const int64_t t0 = seg * kConvSeg;
+  const int64_t left = a.tokens - t0;
+  const uint16_t* v = a.value + b * a.vs_b + c;
+  double w[4][4];
+  {
+    const u16x4* wp = (const u16x4*)(a.weight + c * 4);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const u16x4 ww = wp[q];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[q][j] = (double)h2f(ww[j]);
+    }
+  }
+  u16x4 bias;
+  if (a.bias) bias = *(const u16x4*)(a.bias + c);
+  // in[k] is token t0 - 3 + k; `first` of the three before t0 do not exist
+  u16x4 in[3 + kConvSeg];
+  uint16_t* win = a.window + b * a.ws_b + c;
+  int first = 0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) in[k] = 0;
+  if (seg) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) in[k] = *(const u16x4*)(v + (t0 - 3 + k) * a.vs_l);
+  } else if (a.history) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) in[k] = *(const u16x4*)(win + (k + 1) * a.ws_t);
+  } else {
+    first = 3;
+  }
+#pragma unroll
+  for (int k = 0; k < kConvSeg; ++k)
+    in[3 + k] = *(const u16x4*)(v + (t0 + (k < left ? k : left - 1)) * a.vs_l);
+  if (!seg) {
+    // the only thread of this batch row and these channels that reads the
+    // window also writes it: inputs tokens - 4 .. tokens - 1
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t t = a.tokens - 4 + k;
+      u16x4 last = t == -3 ? in[0] : t == -2 ? in[1] : in[2];
+      if (t >= 0) last = *(const u16x4*)(v + t * a.vs_l);
+      *(u16x4*)(win + k * a.ws_t) = last;
+    }
+  }
+  int part = 0;
+  if (c >= a.n[0]) { c -= a.n[0]; part = 1; }
+  if (part && c >= a.n[1]) { c -= a.n[1]; part = 2; }
+  const int64_t pitch = part == 0 ? a.n[0] : part == 1 ? a.n[1] : a.n[2];
+  uint16_t* o = (part == 0 ? a.out[0] : part == 1 ? a.out[1] : a.out[2]) + (b * a.tokens + t0) * pitch + c;
+#pragma unroll
+  for (int k = 0; k < kConvSeg; ++k) {
+    if (k >= left) break;
+    u16x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double acc = 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double next = __builtin_fma((double)h2f(in[k + q][j]), w[j][q], acc);
+        acc = k + q < 3 && k + q < first ? acc : next;
+      }
+      float s = h2f(f2h((float)acc));
+      if (a.bias) s = h2f(f2h(s + h2f(bias[j])));
+      r[j] = f2h(s / (1.0f + expf(-s)));
+    }
+    *(u16x4*)(o + k * pitch) = r;
+  }
+}
+
+}  // namespace m2r
+
+extern "C" int m2r_causal_conv_tokens(void* window, int64_t ws_b, int64_t ws_t, int history, const void* value,
+                                      int64_t vs_b, int64_t vs_l, const void* weight, const void* bias, void* x,
+                                      void* bm, void* cm, int64_t n_x, int64_t n_b, int64_t n_c, int64_t batch,
+                                      int64_t tokens, int width, hipStream_t stream) {
+  if (batch <= 0 || tokens <= 0 || n_x <= 0 || n_b <= 0 || n_c <= 0) return m2r_fail("conv tokens: non-positive shape");
+  if (width != 4) return m2r_fail("conv tokens: the Mamba-2 convolution width is 4");
+  const int64_t lim = (int64_t)1 << 30;
+  if (batch > lim || tokens > lim || n_x > lim || n_b > lim || n_c > lim)
+    return m2r_fail("conv tokens: size limits");
+  const int64_t channels = n_x + n_b + n_c, segs = (tokens + kConvSeg - 1) / kConvSeg;
+  if ((n_x | n_b | n_c) & 3) return m2r_fail("conv tokens: channel counts must be multiples of 4");
+  if (((ws_b | ws_t | vs_b | vs_l) & 3) || ws_t < channels || vs_l < channels)
+    return m2r_fail("conv tokens: strides must be multiples of 4 elements, the rows' at least the channel count");
+  if (!window || !value || !weight || !x || !bm || !cm) return m2r_fail("conv tokens: null pointer");
+  for (const void* p : {(const void*)window, value, weight, bias, (const void*)x, (const void*)bm, (const void*)cm})
+    if ((uintptr_t)p & 7) return m2r_fail("conv tokens: operands must be 8-byte aligned");
+  const __int128 blocks = ((__int128)(channels / 4) * segs * batch + 255) / 256;
+  if (blocks > 0x7fffffff) return m2r_fail("conv tokens: grid limits exceeded");
+  ConvArgs a{(uint16_t*)window, ws_b, ws_t, (const uint16_t*)value, vs_b, vs_l, (const uint16_t*)weight,
+             (const uint16_t*)bias, {(uint16_t*)x, (uint16_t*)bm, (uint16_t*)cm}, {n_x, n_b, n_c}, batch, tokens,
+             segs, history != 0};
+  hipLaunchKernelGGL(k_conv_tokens, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  return m2r_check(hipGetLastError(), "conv tokens launch");
+}
+
+// ---------------------------------------------------------------------------
 // Gated RMS norm of the Mamba-2 mixer (mamba_ssm's RMSNormGated with
 // norm_before_gate = False, which the reference's controllers call as
 // mx.norm(y, z), mamba2_recall/state_quant.py:298-300), per group of
@@ -74,8 +216,6 @@ extern "C" int m2r_causal_conv_update(void* window, int64_t ws_b, int64_t ws_c, 
 // (per thread in chunk order, then the wave's adjacent-pair butterfly, then
 // the four waves in order), so results do not vary from run to run.
 namespace m2r {
-
-typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void k_gated_rmsnorm(const uint16_t* y, int64_t ys, const uint16_t* z, int64_t zs,
                                                        const uint16_t* weight, uint16_t* out, int64_t os, int gs,

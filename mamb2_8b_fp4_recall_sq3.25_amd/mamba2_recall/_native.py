@@ -42,6 +42,7 @@ _SIGNATURES = {
     "m2r_probe_butterfly": ([P, P, P], I),
     "m2r_set_step_shape": ([I, I], I),
     "m2r_causal_conv_update": ([P, I64, I64, I64, P, I64, P, P, P, I64, I64, I, I, P], I),
+    "m2r_causal_conv_tokens": ([P, I64, I64, I, P, I64, I64, P, P, P, P, P, I64, I64, I64, I64, I64, I, P], I),
     "m2r_gated_rmsnorm": ([P, I64, P, I64, P, P, I64, I64, I64, I64, F32, P], I),
     "m2r_fp4_gemv_g16": ([P, P, P, P, I64, P, I64, I64, I64, I64, P], I),
     "m2r_state_step_ridge_layers_workspace": ([I], I64),

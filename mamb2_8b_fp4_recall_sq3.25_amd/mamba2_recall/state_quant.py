@@ -24,6 +24,7 @@ from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch import nn
 
 from . import _native, fp4, state_codec
 
@@ -88,6 +89,56 @@ def conv_update(window, value, weight, bias, *, silu=True):
                  _native.ptr(value), value.stride(0), _native.ptr(weight), _native.ptr(bias), _native.ptr(out),
                  batch, channels, 4, 1 if silu else 0, _native.stream_of(value))
     return out
+
+
+def _plain(module, cls):
+    """True when calling `module` is exactly cls.forward: its own class, no
+    hooks on it or on all modules, no forward set on the instance."""
+    everywhere = nn.modules.module
+    return (type(module) is cls
+            and not any(name in vars(module) for name in ("forward", "_conv_forward", "_call_impl", "_compiled_call_impl"))
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks or everywhere._global_forward_hooks
+                     or everywhere._global_forward_pre_hooks or everywhere._global_backward_hooks
+                     or everywhere._global_backward_pre_hooks))
+
+
+def conv_tokens_supported(conv, act, value, window, sizes):
+    """Whether conv_tokens computes act(conv(...)): a plain depthwise
+    nn.Conv1d of width 4 and a plain nn.SiLU, FP16 operands on one device in
+    the layouts that the kernel reads, and no autocast.  Anything else runs
+    the modules."""
+    if not (_plain(conv, nn.Conv1d) and _plain(act, nn.SiLU)) or torch.is_autocast_enabled("cuda"):
+        return False
+    channels = sum(sizes)
+    operands = [conv.weight] if conv.bias is None else [conv.weight, conv.bias]
+    return (conv.kernel_size == (4,) and conv.padding == (3,) and conv.stride == (1,) and conv.dilation == (1,)
+            and conv.groups == channels == value.shape[-1] and conv.padding_mode == "zeros"
+            and tuple(conv.weight.shape) == (channels, 1, 4) and tuple(window.shape) == (value.shape[0], channels, 4)
+            and all(type(t) is nn.Parameter and t.is_contiguous() for t in operands)
+            and type(value) is torch.Tensor and value.is_cuda
+            and all(t.dtype == torch.float16 and t.device == value.device and t.data_ptr() % 8 == 0
+                    for t in operands + [value, window])
+            and value.stride(2) == 1 and value.stride(1) >= channels and window.stride(1) == 1
+            and window.stride(2) >= channels
+            and not any(n % 4 for n in tuple(sizes) + value.stride()[:2] + (window.stride(0), window.stride(2))))
+
+
+def conv_tokens(window, value, weight, bias, sizes, *, history):
+    """Causal convolution and SiLU of `value` [B, tokens, C] after the last
+    three inputs of `window` [B, C, 4] (with `history`), in one HIP kernel;
+    the window then holds the last four inputs, zeros before them.  Returns
+    the channel ranges of `sizes` as contiguous tensors.  The convolution's
+    sum and its sum with the bias are each rounded to FP16, as the modules
+    round them."""
+    batch, tokens = value.shape[:2]
+    parts = [torch.empty((batch, tokens, n), dtype=torch.float16, device=value.device) for n in sizes]
+    with torch.cuda.device(value.device):
+        _native.call("m2r_causal_conv_tokens", _native.ptr(window), window.stride(0), window.stride(2),
+                     1 if history else 0, _native.ptr(value), value.stride(0), value.stride(1), _native.ptr(weight),
+                     _native.ptr(bias), *map(_native.ptr, parts), *sizes, batch, tokens, 4,
+                     _native.stream_of(value))
+    return parts
 
 
 def _row_view(t, channels):
@@ -453,8 +504,11 @@ class _MixerController:
         else:
             zxbcdt = mx.in_proj(u)
         z, xbc, dt = torch.split(zxbcdt, self._in_sizes, dim=-1)
-        xbc = self._conv_step(mx, xbc[:, 0], layer)[:, None] if step else self._conv_prefill(mx, xbc, layer)
-        x, bm, cm = torch.split(xbc, self._conv_sizes, dim=-1)
+        if step:
+            parts = torch.split(self._conv_step(mx, xbc[:, 0], layer)[:, None], self._conv_sizes, dim=-1)
+        else:
+            parts = self._conv_prefill(mx, xbc, layer)
+        x, bm, cm = parts
         y, stats = self._scan_layer(index, mx, x.reshape(batch, tokens, self.HEADS, self.HEADDIM), dt,
                                     self._decay_rates(index, mx),
                                     bm.reshape(batch, tokens, self.GROUPS, self.D_STATE),
@@ -537,7 +591,8 @@ class _MixerController:
     # ---------------------------------------------------------------- convolution
     # Same arithmetic as the reference's _convolution (state_quant.py:283-317):
     # mamba_ssm's fused kernels when present, otherwise its PyTorch fallback
-    # (the one-token update as the HIP kernel conv_update).
+    # (the one-token update as the HIP kernel conv_update, several tokens as
+    # the HIP kernel conv_tokens with the modules' results bit for bit).
     def _conv_step(self, mx, column, layer):
         """One token: shift the cached window, append `column` [B, C], return
         the activated convolution output [B, C]."""
@@ -550,10 +605,13 @@ class _MixerController:
     def _conv_prefill(self, mx, xbc, layer):
         """Several tokens (or the first): the causal convolution over the
         cached history (the window's last D_CONV - 1 raw inputs, after the
-        first call) followed by the new inputs; the window then holds the last
-        D_CONV raw inputs, zero-padded on the left."""
+        first call) followed by the new inputs, split into (x, B, C); the
+        window then holds the last D_CONV raw inputs, zero-padded on the left."""
         _, fused_op = _native_conv_ops()
         tokens = xbc.shape[1]
+        if fused_op is None and conv_tokens_supported(mx.conv1d, mx.act, xbc, layer.conv, self._conv_sizes):
+            return conv_tokens(layer.conv, xbc, mx.conv1d.weight, mx.conv1d.bias, self._conv_sizes,
+                               history=layer.tokens > 0)
         fresh = xbc.transpose(1, 2)                              # [B, C, tokens]
         history = self.D_CONV - 1 if layer.tokens > 0 else 0
         series = torch.cat((layer.conv[:, :, 1:], fresh), dim=-1) if history else fresh
@@ -566,7 +624,7 @@ class _MixerController:
                            seq_idx=None).transpose(1, 2)
         else:
             out = mx.act(mx.conv1d(series).transpose(1, 2)[:, :series.shape[-1]])
-        return out[:, history:history + tokens]
+        return torch.split(out[:, history:history + tokens], self._conv_sizes, dim=-1)
 
     # ---------------------------------------------------------------- statistics
     def _accumulate_statistics(self, index, stats, batch, length):

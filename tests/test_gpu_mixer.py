@@ -130,3 +130,79 @@ def test_gated_rmsnorm_three_dim_rows_and_rejections(device):
         gated_rmsnorm(y.transpose(0, 1), z.transpose(0, 1), w, 1e-5, 1024)
     with pytest.raises(RuntimeError, match="group size"):
         gated_rmsnorm(y, z, w, 1e-5, 1000)
+
+
+def conv_modules(sizes, with_bias, device, gen):
+    channels = sum(sizes)
+    conv = nn.Conv1d(channels, channels, 4, groups=channels, padding=3, bias=with_bias).to(device).half()
+    with torch.no_grad():
+        conv.weight.copy_(torch.randn(channels, 1, 4, generator=gen, device=device) * 0.5)
+        if with_bias:
+            conv.bias.copy_(torch.randn(channels, generator=gen, device=device) * 0.1)
+    return conv.requires_grad_(False)
+
+
+@pytest.mark.parametrize("sizes", [(8192, 1024, 1024), (28, 4, 16)])
+@pytest.mark.parametrize("batch,tokens,history,with_bias,scale", [
+    (1, 1, False, True, 1.0), (2, 1, True, True, 1.0), (3, 2, True, False, 30.0), (2, 3, False, True, 1.0),
+    (1, 4, False, True, 1e-4), (1, 7, True, True, 1.0), (2, 8, False, False, 1.0), (1, 9, True, True, 1e-7),
+    (3, 37, True, True, 1.0)])
+def test_conv_tokens_bit_exact(device, sizes, batch, tokens, history, with_bias, scale):
+    """Against the sum in binary64 over the taps that exist, rounded through
+    binary32 as the library's convolution does, the binary16 bias and torch's
+    SiLU; no tolerance.  An infinite weight tells a left-out tap from a zero
+    input."""
+    from mamba2_recall.state_quant import conv_tokens, conv_tokens_supported
+    channels = sum(sizes)
+    gen = torch.Generator(device=device).manual_seed(7 * tokens + channels)
+    print(f"[conv tokens] B={batch} L={tokens} C={channels} history={history} bias={with_bias} x{scale}", flush=True)
+    conv = conv_modules(sizes, with_bias, device, gen)
+    conv.weight[3, 0, 0] = float("inf")
+    win = make_window(batch, channels, "time_major", device, gen, scale)
+    projected = (torch.randn(batch, tokens, channels + 136, generator=gen, device=device) * scale).half()
+    value = projected[..., 64:64 + channels]
+    assert conv_tokens_supported(conv, nn.SiLU(), value, win, sizes)
+    past = win[:, :, 1:] if history else win[:, :, :0]
+    series = torch.cat((past, value.transpose(1, 2)), dim=-1).double().cpu().numpy()
+    lead = past.shape[-1]
+    w = conv.weight[:, 0].double().cpu().numpy()
+    acc = np.zeros((batch, channels, tokens))
+    for k in range(4):
+        for t in range(tokens):
+            if lead + t - 3 + k >= 0:
+                with np.errstate(invalid="ignore"):
+                    acc[..., t] += series[..., lead + t - 3 + k] * w[:, k]
+    with np.errstate(over="ignore"):
+        s = torch.from_numpy(acc.astype(np.float32).astype(np.float16)).to(device)
+    if with_bias:
+        s = s + conv.bias[:, None]
+    want = nn.functional.silu(s).transpose(1, 2)
+    want_win = np.concatenate((np.zeros((batch, channels, 4)), series), axis=-1)[..., -4:]
+    got = conv_tokens(win, value, conv.weight, conv.bias, sizes, history=history)
+    assert torch.equal(win.double().cpu(), torch.from_numpy(want_win))
+    for part, ref in zip(got, torch.split(want, sizes, dim=-1)):
+        assert part.is_contiguous() and part.shape == ref.shape
+        same = (part.view(torch.int16) == ref.contiguous().view(torch.int16)) | (part.isnan() & ref.isnan())
+        assert bool(same.all()), f"{int((~same).sum())} outputs differ"
+
+
+def test_conv_tokens_leaves_other_modules_alone(device):
+    from mamba2_recall.state_quant import conv_tokens_supported
+    gen = torch.Generator(device=device).manual_seed(3)
+    sizes = (24, 8, 16)
+    conv, act = conv_modules(sizes, True, device, gen), nn.SiLU()
+    win = make_window(2, 48, "time_major", device, gen, 1.0)
+    value = torch.zeros(2, 5, 64, device=device, dtype=torch.float16)[..., 8:56]
+    assert conv_tokens_supported(conv, act, value, win, sizes)
+    assert not conv_tokens_supported(conv, nn.Identity(), value, win, sizes)
+    assert not conv_tokens_supported(conv, act, value.contiguous().transpose(0, 1), win, sizes)
+    assert not conv_tokens_supported(conv, act, value, win.contiguous(), sizes)
+    assert not conv_tokens_supported(conv, act, torch.zeros(2, 5, 65, device=device, dtype=torch.float16)[..., 1:49],
+                                     win, sizes)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not conv_tokens_supported(conv, act, value, win, sizes)
+    hook = act.register_forward_hook(lambda *_: None)
+    assert not conv_tokens_supported(conv, act, value, win, sizes)
+    hook.remove()
+    conv.forward = lambda x: x
+    assert not conv_tokens_supported(conv, act, value, win, sizes)
