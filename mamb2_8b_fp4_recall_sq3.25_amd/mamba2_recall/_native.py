@@ -6,6 +6,7 @@ into it and raises if it is missing.  There is no CPU or Triton fallback.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from pathlib import Path
 
@@ -96,14 +97,28 @@ def call(name: str, *args):
 
 def ptr(t):
     """Device pointer of a tensor (None -> NULL)."""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
+# An eager one-token scan is bound by the host, the kernel taking under 8 us.
+# Plain integers as pointers, the raw stream and no device switch where the
+# device is already current, with the layout worked out and each storage asked
+# once per call, took it from 33 to 24 us a call.
 def stream_of(t: torch.Tensor):
     """The current HIP stream of `t`'s device, as the C-ABI expects it."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if not t.is_cuda:
+        return torch.cuda.current_stream(t.device).cuda_stream   # raises
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_HERE = contextlib.nullcontext()
+
+
+def device_of(t: torch.Tensor):
+    """A context with `t`'s device current: nothing where it already is."""
+    if t.is_cuda and t.get_device() == torch.cuda.current_device():
+        return _HERE
+    return torch.cuda.device(t.device)
 
 
 def require_device(t: torch.Tensor, what: str = "tensor"):

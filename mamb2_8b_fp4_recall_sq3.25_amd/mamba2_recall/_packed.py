@@ -53,7 +53,7 @@ def launch_packed(kind, x, dt, A, B, C, D, dt_bias, perm, tensors, *, n8, n4, nz
     db_f32 = int(dt_bias.dtype == torch.float32)
     p = _native.ptr
     stream = _native.stream_of(x)
-    with torch.cuda.device(x.device):
+    with _native.device_of(x):
         common = (p(x), p(dt), p(A), p(B), p(C), p(D), d_f32, p(dt_bias), db_f32, p(perm))
         geo = (batch, length, heads, dim, groups)
         if kind == "ridge":
@@ -93,7 +93,7 @@ def decode_rows(tensors, n8, n4, *, shape):
     out = torch.empty(shape, dtype=torch.float32, device=lo.device)
     batch, heads, dim, _ = shape
     p = _native.ptr
-    with torch.cuda.device(lo.device):
+    with _native.device_of(lo):
         _native.call("m2r_state_decode", 0, n8, n4, 128 - n8 - n4, p(lo), p(hi), p(q4), None, p(s8), p(s4),
                      None, p(out), batch, heads, dim, 0, _native.stream_of(lo))
     return out

@@ -93,7 +93,7 @@ def decode_into(packed, scales, global_scale, out, *, rows, columns, group, err_
     device int32[1] that accumulates the violation bits."""
     p = _native.ptr
     stream = _native.stream_of(packed)
-    with torch.cuda.device(packed.device):
+    with _native.device_of(packed):
         if group == 16:
             _native.call("m2r_fp4_decode_g16", p(packed), p(scales), p(global_scale), p(out), rows, columns,
                          p(err_flag), stream)
@@ -138,7 +138,7 @@ def gemv_g16(packed, scales, global_scale, u, *, out=None):
     if out is None:
         out = torch.empty((rows, n), dtype=torch.float16, device=u.device)
     _need(out.dtype == torch.float16 and tuple(out.shape) == (rows, n) and out.stride(1) == 1, "out must be FP16 [M, N]")
-    with torch.cuda.device(u.device):
+    with _native.device_of(u):
         _native.call("m2r_fp4_gemv_g16", _native.ptr(packed), _native.ptr(sb), _native.ptr(global_scale),
                      _native.ptr(u), u.stride(0), _native.ptr(out), out.stride(0), rows, n, columns,
                      _native.stream_of(u))

@@ -46,24 +46,28 @@ def allocate_state(batch, heads, dim, dstate, device, *, layout):
 
 def validate_state(state, device, layout):
     """fp4_zero_predictor_codec_v1.py:52-73."""
-    spec = layout_descriptor(layout)
+    return _validate_state(state, torch.device(device), layout, layout_descriptor(layout))
+
+
+def _validate_state(state, device, layout, spec):
     if (state.mode != "latent_fp8_" + layout or len(state.shape) != 4 or state.shape[-1] != 128
             or set(state.tensors) != {"lo", "hi", "q4", "latent", "s8", "s4"}):
         raise ValueError("Latent packed state mode/inventory differs")
     base = tuple(state.shape[:3])
     if min(base) <= 0:
         raise ValueError("Invalid latent state geometry")
-    storages = set()
+    storages, total = set(), 0
     for name, value in state.tensors.items():
         shape = base + ((spec["tensor_widths"][name],) if name in spec["tensor_widths"] else ())
         dtype = (torch.float16 if name in ("s8", "s4") else
                  torch.float8_e4m3fn if name == "latent" else torch.uint8)
-        if (tuple(value.shape) != shape or value.dtype != dtype or value.device != torch.device(device)
+        if (value.shape != shape or value.dtype != dtype or value.device != device
                 or not value.is_contiguous() or value.storage_offset() != 0
-                or value.untyped_storage().nbytes() != value.numel() * value.element_size()):
+                or (storage := value.untyped_storage()).nbytes() != value.numel() * value.element_size()):
             raise ValueError("Latent packed state backing allocation differs: " + name)
-        storages.add(value.untyped_storage().data_ptr())
-    if len(storages) != 6 or state.nbytes != base[0] * base[1] * base[2] * 52:
+        storages.add(storage.data_ptr())
+        total += storage.nbytes()
+    if len(storages) != 6 or total != base[0] * base[1] * base[2] * 52:
         raise ValueError("Latent state aliases or exceeds 52-byte row")
     return True
 
@@ -74,7 +78,10 @@ def check_static_metadata(permutation, basis, latent_scale, predictor, *, groups
     permutation, bases, latent scales and predictor.  The kernel indexes these
     tables by the shapes checked here, so every scan runs this, whatever its
     `validate` flag; it reads tensor metadata only and never synchronizes."""
-    spec = layout_descriptor(layout)
+    _check_static_metadata(permutation, basis, latent_scale, predictor, groups, layout_descriptor(layout), device)
+
+
+def _check_static_metadata(permutation, basis, latent_scale, predictor, groups, spec, device):
     if (not all(isinstance(v, torch.Tensor) for v in (permutation, basis, latent_scale, predictor))
             or permutation.dtype != torch.uint8 or tuple(permutation.shape) != (groups, 128)
             or permutation.device != device
@@ -122,19 +129,19 @@ def scan(x, dt, A, B, C, D, dt_bias, state, permutation, basis, latent_scale, pr
     batch, length, heads, dim = x.shape
     if length < 1 or dim % RP or state.shape != (batch, heads, dim, 128):
         raise ValueError("Positive sequence and matching latent state required")
-    validate_state(state, x.device, layout)
+    device = x.device
+    _validate_state(state, device, layout, spec)
     groups = B.shape[2] if B.ndim == 4 else 0
     expected = ((dt, (batch, length, heads)), (A, (heads,)), (B, (batch, length, groups, 128)),
                 (C, (batch, length, groups, 128)), (D, (heads,)), (dt_bias, (heads,)))
     for value, shape in expected:
-        if tuple(value.shape) != shape or value.device != x.device:
+        if value.shape != shape or value.device != device:
             raise ValueError("Latent scan input geometry/device differs")
     if (groups < 1 or heads % groups or A.dtype != torch.float32
             or any(v.dtype != torch.float16 for v in (dt, B, C))
             or any(v.dtype not in (torch.float16, torch.float32) for v in (D, dt_bias))):
         raise ValueError("Latent scan dtype/grouping differs")
-    check_static_metadata(permutation, basis, latent_scale, predictor, groups=groups, layout=layout,
-                          device=x.device)
+    _check_static_metadata(permutation, basis, latent_scale, predictor, groups, spec, device)
     if validate:
         validate_statics(permutation, basis, latent_scale, predictor, groups=groups, layout=layout,
                          device=x.device)

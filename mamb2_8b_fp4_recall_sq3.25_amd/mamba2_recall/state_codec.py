@@ -118,7 +118,7 @@ def scan(x, dt, A, B, C, D, dt_bias, state, permutation=None, collect_stats=Fals
     tiles = (p + RP - 1) // RP
     stats = torch.zeros((b, h, tiles, N), device=x.device, dtype=torch.float32) if collect_stats else None
     ptr = _native.ptr
-    with torch.cuda.device(x.device):
+    with _native.device_of(x):
         _native.call("m2r_state_step_s16", ptr(x), ptr(dt), ptr(A), ptr(B), ptr(C), ptr(D),
                      int(D.dtype == torch.float32), ptr(dt_bias), int(dt_bias.dtype == torch.float32),
                      ptr(state.tensors["state"]), ptr(y), ptr(stats), b, length, h, p, g, _native.stream_of(x))
@@ -168,7 +168,7 @@ def encode_state_(state, dense_permuted):
     b, h, p, _ = state.shape
     t = state.tensors
     ptr = _native.ptr
-    with torch.cuda.device(v.device):
+    with _native.device_of(v):
         _native.call("m2r_state_encode_legacy", ptr(v), ptr(t["lo"]), ptr(t["hi"]), ptr(t["q4"]), ptr(t["s8"]),
                      ptr(t["s4"]), b * h * p, _native.stream_of(v))
     return state

@@ -112,7 +112,7 @@ def scan(x, dt, A, B, C, D, dt_bias, state, table, table_kind="permutation"):
     x, dt, A, B, C, D, dt_bias, table = (v.contiguous() for v in (x, dt, A, B, C, D, dt_bias, table))
     out = torch.empty_like(x)
     ptr = _native.ptr
-    with torch.cuda.device(x.device):
+    with _native.device_of(x):
         _native.call("m2r_state_step_dense3", ptr(x), ptr(dt), ptr(A), ptr(B), ptr(C), ptr(D),
                      int(D.dtype == torch.float32), ptr(dt_bias), int(dt_bias.dtype == torch.float32), ptr(table),
                      int(table_kind == "equalizer"), ptr(state.tensors["codes"]), ptr(state.tensors["scales"]),
@@ -128,7 +128,7 @@ def decode_state(state, table=None, table_kind="permutation"):
     b, h, p, _ = state.shape
     value = torch.empty(state.shape, dtype=torch.float32, device=codes.device)
     ptr = _native.ptr
-    with torch.cuda.device(codes.device):
+    with _native.device_of(codes):
         _native.call("m2r_state_decode", 1, 0, 0, 0, ptr(codes), None, None, None, ptr(state.tensors["scales"]),
                      None, None, ptr(value), b, h, p, 0, _native.stream_of(codes))
     if table is None:

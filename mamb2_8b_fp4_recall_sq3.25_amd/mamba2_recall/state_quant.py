@@ -133,7 +133,7 @@ def conv_tokens(window, value, weight, bias, sizes, *, history):
     round them."""
     batch, tokens = value.shape[:2]
     parts = [torch.empty((batch, tokens, n), dtype=torch.float16, device=value.device) for n in sizes]
-    with torch.cuda.device(value.device):
+    with _native.device_of(value):
         _native.call("m2r_causal_conv_tokens", _native.ptr(window), window.stride(0), window.stride(2),
                      1 if history else 0, _native.ptr(value), value.stride(0), value.stride(1), _native.ptr(weight),
                      _native.ptr(bias), *map(_native.ptr, parts), *sizes, batch, tokens, 4,
