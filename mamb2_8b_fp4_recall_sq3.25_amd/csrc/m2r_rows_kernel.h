@@ -23,8 +23,9 @@
 //    (eight lanes: one token ahead).  dt activations are evaluated 64 tokens
 //    at a time.
 // 512 tokens of a batch-1 layer, against the several waves per 64-row slot
-// and (dense rows) one lane per row before: ridge 24/44/60 626 -> 300 us,
-// tier 32/32/64 594 -> 230, legacy 648 -> 250, dense3 2,069 -> 300.
+// and (dense rows) one lane per row before: ridge 24/44/60 629 -> 328 us
+// (the records kernel included), tier 32/32/64 596 -> 264, legacy 651 -> 270,
+// dense3 2,049 -> 337.
 // The arithmetic is that of m2r_step.h and m2r_dense3.hip: codes and scales
 // equal a call per token bit for bit, and so does a ridge row's y, whose
 // one-token step sums in the same order (the other codecs' y differ from it
