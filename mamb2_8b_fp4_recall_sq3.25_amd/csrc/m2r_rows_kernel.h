@@ -560,7 +560,8 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads) {
       bool unclamped = finite_in, zero[SETS];
 #pragma unroll
       for (int e = 0; e < SETS; ++e) {
-        zero[e] = !DEN32 && stored[e] == 0.f;
+        // a stored scale that is zero (underflowed) or infinite: code 0
+        zero[e] = !DEN32 && (!(stored[e] > 0.f) || stored[e] == __builtin_inff());
         unclamped = unclamped && (DEN32 || zero[e] || stored[e] >= 0x1p-14f);
       }
       if (__builtin_amdgcn_ballot_w64(!unclamped) == 0) {

@@ -93,16 +93,29 @@ def assert_y_pattern_close(y_dev, y_ref, what):
     assert err <= Y_TOL, f"{what}: y rel L2 {err:.3e} > {Y_TOL}"
 
 
+def overflow_scales(inp, tokens):
+    """At `tokens`, finite inputs whose updates are finite but overflow a
+    tier's binary16 stored scale (7 * 65504 in the INT4 tier, 127 * 65504 in
+    the INT8 one): both tiers' on every third head, about the INT4 tier's
+    alone on the next ones."""
+    for t in tokens:
+        inp["x"][:, t, 0::3] = cases.f16(np.float32(6e4))
+        inp["x"][:, t, 1::3] = cases.f16(np.float32(1e4))
+        inp["dt"][:, t] = cases.f16(np.float32(6.0))
+        inp["B"][:, t] = cases.f16(cases.f16_to_f32(inp["B"][:, t]) * 40.0)
+
+
 NONFINITE_SCALES = [0x7C00, 0xFC00, 0x7E00, 0x7C00, 0xFE00, 0x7C00]
 
 
 def run_ridge(oracle, device, layout, batch, L, H, P, G, seed, *, random_state=True, d_f32=False, db_f32=False,
-              dt_bias_zero=True, x_scale=1.0, scale_mu=-4.0, special_scales=None, shifted=()):
+              dt_bias_zero=True, x_scale=1.0, scale_mu=-4.0, special_scales=None, shifted=(), overflow=()):
     from mamba2_recall import ridge_codec
     n8, n4, nz = ridge_counts(layout)
     rng = np.random.default_rng(seed)
     inp = cases.step_inputs(rng, batch, L, H, P, G, d_f32=d_f32, db_f32=db_f32, dt_bias_zero=dt_bias_zero,
                             x_scale=x_scale)
+    overflow_scales(inp, overflow)
     sta = cases.ridge_statics(rng, G, n8, n4, nz)
     st0 = (cases.random_packed_state(rng, batch, H, P, n8, n4, latent=True, scale_mu=scale_mu) if random_state
            else cases.zero_packed_state(batch, H, P, n8, n4, latent=True))
@@ -122,18 +135,19 @@ def run_ridge(oracle, device, layout, batch, L, H, P, G, seed, *, random_state=T
                             pred, layout=layout)
     torch.cuda.synchronize()
     assert_state_equal(from_state(state), ref_state, f"ridge {layout}")
-    if special_scales is not None:
+    if special_scales is not None or overflow:
         return assert_y_pattern_close(y, y_ref, f"ridge {layout}")
     return assert_y_close(y, y_ref, f"ridge {layout}")
 
 
 def run_tier(oracle, device, kind, layout, batch, L, H, P, G, seed, *, random_state=True, d_f32=False,
-             db_f32=False, dt_bias_zero=True, x_scale=1.0, scale_mu=-4.0, special_scales=None, shifted=()):
+             db_f32=False, dt_bias_zero=True, x_scale=1.0, scale_mu=-4.0, special_scales=None, shifted=(), overflow=()):
     from mamba2_recall import state_codec, tier_codec
     n8, n4, nz = tier_counts(layout)
     rng = np.random.default_rng(seed)
     inp = cases.step_inputs(rng, batch, L, H, P, G, d_f32=d_f32, db_f32=db_f32, dt_bias_zero=dt_bias_zero,
                             x_scale=x_scale)
+    overflow_scales(inp, overflow)
     st0 = (cases.random_packed_state(rng, batch, H, P, n8, n4, scale_mu=scale_mu) if random_state
            else cases.zero_packed_state(batch, H, P, n8, n4))
     if special_scales is not None:
@@ -156,7 +170,7 @@ def run_tier(oracle, device, kind, layout, batch, L, H, P, G, seed, *, random_st
                                layout=layout)
     torch.cuda.synchronize()
     assert_state_equal(from_state(state), ref_state, f"{kind} {layout}")
-    if special_scales is not None:
+    if special_scales is not None or overflow:
         return assert_y_pattern_close(y, y_ref, f"{kind} {layout}")
     return assert_y_close(y, y_ref, f"{kind} {layout}")
 
@@ -696,6 +710,18 @@ def test_rows_scan_unusual_states(oracle, device, batch, L):
     run_dense3(oracle, device, "permutation", batch, L, H, P, G, 3451, x_scale=1e-9, scale_mu=-24.0)
     run_dense3(oracle, device, "equalizer", batch, L, H, P, G, 3452, special_scales=NONFINITE_SCALES,
                nonfinite_y=True)
+
+
+@pytest.mark.parametrize("batch,L", [(1, 24), (5, 24), (8, 24), (13, 64)])
+def test_rows_scan_stored_scales_overflow(oracle, device, batch, L):
+    """A tier's stored scale that overflows binary16 from finite inputs, at a
+    middle and at the last token, on 8, 4, 2 and 1 or 4 lanes per row: code 0,
+    as the reference's quotient by infinity gives."""
+    H, P, G = 128, 16, 8
+    for i, layout in enumerate(("24_48_56", "8_80_40")):
+        run_ridge(oracle, device, layout, batch, L, H, P, G, 3500 + i, overflow=(9, L - 1))
+        run_tier(oracle, device, "tier", layout, batch, L, H, P, G, 3510 + i, overflow=(9, L - 1))
+    run_tier(oracle, device, "legacy", "16_64_48", batch, L, H, P, G, 3520, overflow=(9, L - 1))
 
 
 def run_s16(oracle, device, batch, L, H, P, G, seed, collect):
