@@ -556,9 +556,10 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
     const uint16_t* p0 = s_pred + f0 * NZ;
     const uint16_t* p1 = s_pred + f1 * NZ;
     // every LDS read of a half is issued before its first use; four partial
-    // sums per output (readout-only value: summation order free)
+    // sums per half and output, folded as the split form above folds them, so
+    // that every workgroup shape has the same corrections
     constexpr int Q = NZ / 4, QH = (Q + 1) / 2;
-    float a0[4] = {0.f, 0.f, 0.f, 0.f}, a1[4] = {0.f, 0.f, 0.f, 0.f};
+    float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       f32x4 cv[QH];
@@ -571,6 +572,7 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
         if constexpr (F > 64) w1[i] = *(const uint2*)(p1 + d);
       }
       __builtin_amdgcn_sched_barrier(0);
+      float a0[4] = {0.f, 0.f, 0.f, 0.f}, a1[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < QH; ++i) {
         if (h * QH + i >= Q) break;
@@ -585,9 +587,10 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
           a1[3] = __builtin_fmaf(cv[i].w, h2f((uint16_t)(w1[i].y >> 16)), a1[3]);
         }
       }
+      const float part0 = (a0[0] + a0[1]) + (a0[2] + a0[3]), part1 = (a1[0] + a1[1]) + (a1[2] + a1[3]);
+      acc0 = h ? acc0 + part0 : part0;
+      acc1 = h ? acc1 + part1 : part1;
     }
-    const float acc0 = (a0[0] + a0[1]) + (a0[2] + a0[3]);
-    const float acc1 = (a1[0] + a1[1]) + (a1[2] + a1[3]);
     if (lane < NL) wt.cw[lane] = c0 + acc0;
     if (64 + lane < NL) wt.cw[64 + lane] = c1 + acc1;
     // correction of the latent coefficients: outputs NL and NL + 1

@@ -272,15 +272,12 @@ def forced_shape(request):
 
 @pytest.mark.parametrize("L", [1, 3])
 def test_ridge_every_shape_same_bits(device, L):
-    """Every workgroup shape of four or eight waves, including the slots on
-    two and four waves (whose waves step parts of a tier and share the tier
-    maxima and the readout partial sums), gives the same codes, scales and y
-    bit for bit: the readout is summed per segment of the carried coordinates
-    in one fixed order, and the ridge correction is split the same way.  (The
-    one-wave workgroups compute the correction of the readout weights in
-    another order: the same codes, y within the oracle tolerance, checked by
-    the per-shape tests.)  Layouts whose INT4 tier is split between waves,
-    whose INT8 tier is, and neither."""
+    """Every workgroup shape, including the slots on two and four waves
+    (whose waves step parts of a tier and share the tier maxima and the
+    readout partial sums), gives the same codes, scales and y bit for bit: the
+    readout is summed per half segment of the carried coordinates in one fixed
+    order, and so is the ridge correction.  Layouts whose INT4 tier is split
+    between waves, whose INT8 tier is, and neither."""
     from mamba2_recall import _native, ridge_codec
     for layout in ("8_80_40", "24_48_56", "36_24_68", "44_8_76"):
         n8, n4, nz = ridge_counts(layout)
@@ -294,7 +291,7 @@ def test_ridge_every_shape_same_bits(device, L):
         basis, ls, pred = (dev16(sta[k], device) for k in ("basis", "lscale", "pred"))
         results = []
         try:
-            for shape in [sh for sh in SHAPES if sh[0] >= 4]:
+            for shape in SHAPES:
                 print(f"[same bits] layout={layout} L={L} shape={shape}", flush=True)
                 _native.call("m2r_set_step_shape", *shape)
                 state = ridge_codec.allocate_state(B, H, P, 128, device, layout=layout)
@@ -373,6 +370,38 @@ def test_ridge_token_records_same_bits_as_in_kernel_build(device, layout):
                 assert not torch.isnan(ws).all()   # the records path ran
     finally:
         _native.call("m2r_set_step_shape", 0, 0)
+
+
+@pytest.mark.parametrize("batch,H,G", [(8, 128, 8), (10, 128, 8), (13, 128, 8), (20, 60, 10), (60, 9, 3),
+                                       (200, 9, 3)])
+@pytest.mark.parametrize("layout", ["24_48_56", "8_80_40"])
+def test_ridge_workspace_same_bits_as_without(device, layout, batch, H, G):
+    """With and without a workspace, the same codes, scales, latent bytes and
+    y, at 1,024, 1,280 and 1,664 slots of the model's 16 heads per group (two,
+    four and one or four lanes per row) and where the step without a workspace
+    runs one wave per workgroup: 6 heads per group at 1,200 slots, 3 at 540
+    and 1,800."""
+    from mamba2_recall import _native, ridge_codec
+    n8, n4, nz = ridge_counts(layout)
+    L, P = 17, 16
+    print(f"[ridge workspace] layout={layout} B={batch} H={H} G={G}", flush=True)
+    rng = np.random.default_rng(770 + batch)
+    inp = cases.step_inputs(rng, batch, L, H, P, G)
+    sta = cases.ridge_statics(rng, G, n8, n4, nz)
+    st0 = cases.random_packed_state(rng, batch, H, P, n8, n4, latent=True)
+    t = device_inputs(inp, device)
+    perm = torch.from_numpy(inp["perm"]).to(device)
+    basis, ls, pred = (dev16(sta[k], device) for k in ("basis", "lscale", "pred"))
+    ws = torch.empty(int(_native.lib().m2r_ridge_records_bytes(batch, L, G)) // 4, dtype=torch.float32, device=device)
+    out = []
+    for w in (None, ws):
+        state = ridge_codec.allocate_state(batch, H, P, 128, device, layout=layout)
+        to_state(st0, state, device)
+        y = _ridge_step_direct(t, perm, basis, ls, pred, state, layout, w)
+        out.append(dict({k: v.view(torch.uint8) for k, v in state.tensors.items()}, y=y.view(torch.int16)))
+    for k in out[0]:
+        differ = int((out[0][k] != out[1][k]).sum())
+        assert differ == 0, f"{k}: {differ} of {out[0][k].numel()} differ"
 
 
 def test_ridge_token_records_graph_replays_match_eager(device):
