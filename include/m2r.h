@@ -104,7 +104,7 @@ int m2r_state_step_legacy(const void* x, const void* dt, const float* A, const v
  * slot (each wave steps a quarter of the carried coordinates); (0,0) restores
  * the automatic choice.  A forced shape whose head count does not divide the heads per group
  * falls back to the automatic choice.  A forced shape also keeps multi-token calls on the one-lane-per-row
- * kernels, except (4,0), (4,-2) and (4,-4) with a ridge workspace.  Process-wide; results do not depend on the shape.  No counterpart
+ * kernels, with a ridge workspace too (which they do not use).  Process-wide; results do not depend on the shape.  No counterpart
  * in the reference (its Triton launch grid is fixed per call).
  */
 int m2r_set_step_shape(int waves_per_block, int heads_per_wave);

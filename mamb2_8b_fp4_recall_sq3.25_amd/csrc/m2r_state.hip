@@ -54,11 +54,10 @@ static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   // Several tokens: the row-split scan, where rows, inputs and readouts are
   // whole 16-byte pieces: a ridge launch that brings a workspace for its token
   // records, another where the scan pays (m2r_rows.hip).  A forced shape keeps
-  // it away, but the shapes of several waves per slot take token records.
-  const bool rows_ok = a.L > 1 && (a.dma_tiles & 1) &&
+  // it away.
+  const bool rows_ok = !forced && a.L > 1 && (a.dma_tiles & 1) &&
                        (((uintptr_t)a.x | (uintptr_t)a.Bm | (uintptr_t)a.Cm | (uintptr_t)a.y) & 15) == 0;
-  const bool rows = MODE == MODE_RIDGE ? a.rec && (!forced || forced == 4 * 16 || forced == FOUR_PER_SLOT)
-                                       : !forced && rows_scan_pays(MODE, N8 + N4, slots, a.L);
+  const bool rows = MODE == MODE_RIDGE ? a.rec != nullptr : rows_scan_pays(MODE, N8 + N4, slots, a.L);
   if (rows_ok && rows)
     return launch_rows<N8, N4, NZ, MODE>(a, stream);
   if (forced == 4 * 16 && hpg % 2 == 0) {   // (4, 0): two waves per head slot

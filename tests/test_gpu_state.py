@@ -270,14 +270,15 @@ def forced_shape(request):
     _native.call("m2r_set_step_shape", 0, 0)
 
 
-@pytest.mark.parametrize("L", [1, 3])
+@pytest.mark.parametrize("L", [1, 3, 17])
 def test_ridge_every_shape_same_bits(device, L):
     """Every workgroup shape, including the slots on two and four waves
     (whose waves step parts of a tier and share the tier maxima and the
     readout partial sums), gives the same codes, scales and y bit for bit: the
     readout is summed per half segment of the carried coordinates in one fixed
     order, and so is the ridge correction.  Layouts whose INT4 tier is split
-    between waves, whose INT8 tier is, and neither."""
+    between waves, whose INT8 tier is, and neither.  17 tokens with the
+    automatic shape run the row-split scan."""
     from mamba2_recall import _native, ridge_codec
     for layout in ("8_80_40", "24_48_56", "36_24_68", "44_8_76"):
         n8, n4, nz = ridge_counts(layout)
@@ -291,7 +292,7 @@ def test_ridge_every_shape_same_bits(device, L):
         basis, ls, pred = (dev16(sta[k], device) for k in ("basis", "lscale", "pred"))
         results = []
         try:
-            for shape in SHAPES:
+            for shape in SHAPES + [(0, 0)]:
                 print(f"[same bits] layout={layout} L={L} shape={shape}", flush=True)
                 _native.call("m2r_set_step_shape", *shape)
                 state = ridge_codec.allocate_state(B, H, P, 128, device, layout=layout)
@@ -329,14 +330,15 @@ def _ridge_step_direct(t, perm, basis, ls, pred, state, layout, ws):
 
 @pytest.mark.parametrize("layout", RIDGE_LAYOUTS)
 def test_ridge_token_records_same_bits_as_in_kernel_build(device, layout):
-    """Multi-token launches of the shapes with several waves per slot read
-    their tokens' state-independent values from records a first kernel wrote
-    (the split token build of four waves, run per token): codes, scales,
-    latent bytes and y equal the in-kernel build's bit for bit, with the
-    automatic shape (four or two waves per slot) and forced two- and four-wave
-    slots, token counts that are and are not multiples of the records
-    kernel's 8 tokens per workgroup, batch rows 1 to 3, and a ragged head
-    dimension (P = 72: a second, partly filled 64-row block per head)."""
+    """Multi-token launches with a workspace read their tokens'
+    state-independent values from records a first kernel wrote (the split
+    token build of four waves, run per token): codes, scales, latent bytes and
+    y equal the in-kernel build's bit for bit, of the automatic shape (four or
+    two waves per slot) and of forced two- and four-wave slots, token counts
+    that are and are not multiples of the records kernel's 8 tokens per
+    workgroup, batch rows 1 to 3, and a ragged head dimension (P = 72: a
+    second, partly filled 64-row block per head).  A forced shape runs as
+    asked: it leaves the workspace alone."""
     from mamba2_recall import _native, ridge_codec
     n8, n4, nz = ridge_counts(layout)
     H, G = 128, 8
@@ -344,7 +346,6 @@ def test_ridge_token_records_same_bits_as_in_kernel_build(device, layout):
         for shape in ((0, 0), (4, 0), (4, -4)):
             for batch, L, P in ((1, 37, 64), (2, 16, 64), (1, 2, 64), (3, 19, 72)):
                 print(f"[token records] layout={layout} shape={shape} B={batch} L={L} P={P}", flush=True)
-                _native.call("m2r_set_step_shape", *shape)
                 rng = np.random.default_rng(700 + batch * 100 + L)
                 inp = cases.step_inputs(rng, batch, L, H, P, G)
                 sta = cases.ridge_statics(rng, G, n8, n4, nz)
@@ -360,7 +361,11 @@ def test_ridge_token_records_same_bits_as_in_kernel_build(device, layout):
                 s_rec = ridge_codec.allocate_state(batch, H, P, 128, device, layout=layout)
                 to_state(st0, s_build, device)
                 to_state(st0, s_rec, device)
-                y_build = _ridge_step_direct(t, perm, basis, ls, pred, s_build, layout, None)
+                _native.call("m2r_set_step_shape", *shape)
+                y_build = _ridge_step_direct(t, perm, basis, ls, pred, s_build, layout, ws if any(shape) else None)
+                torch.cuda.synchronize()
+                assert torch.isnan(ws).all(), shape
+                _native.call("m2r_set_step_shape", 0, 0)
                 y_rec = _ridge_step_direct(t, perm, basis, ls, pred, s_rec, layout, ws)
                 torch.cuda.synchronize()
                 assert torch.equal(y_rec.view(torch.int16), y_build.view(torch.int16)), (layout, shape, batch, L, P)
