@@ -60,7 +60,7 @@ int m2r_state_step_ridge(const void* x, const void* dt, const float* A, const vo
  * state-independent token values (readout weights with the correction,
  * dead-tier dot products, sum b.c, the carried b) into `workspace`, and the
  * multi-token scan, which spreads each row over one to eight lanes, reads
- * them (faster from 16 to 64 tokens on, by the number of rows).  Results are
+ * them (m2r_scan_lanes says where that is faster).  Results are
  * identical to m2r_state_step_ridge bit for bit.
  * workspace: null (then exactly m2r_state_step_ridge), or 16-byte aligned
  * device memory of at least m2r_ridge_records_bytes(batch, L, G) bytes,
@@ -74,6 +74,16 @@ int m2r_state_step_ridge_ws(const void* x, const void* dt, const float* A, const
                             int64_t workspace_bytes, hipStream_t stream);
 /* Workspace bytes of m2r_state_step_ridge_ws: batch * L * G records of 1 KiB. */
 int64_t m2r_ridge_records_bytes(int64_t batch, int64_t L, int64_t G);
+/*
+ * Lanes per row (8, 4, 2 or 1) of the multi-token scan where it beats the
+ * one-lane-per-row kernels, else 0.  codec: 0 legacy, 1 tier, 2 ridge, 3
+ * dense3; n8, n4 the carried coordinates of a packed row.  The legacy, tier
+ * and dense3 steps follow it for operands on 16-byte boundaries; a ridge step
+ * runs the scan whenever it is given a workspace, so its caller brings one
+ * where this is not 0.  No counterpart in the reference (its scans are one
+ * Triton kernel each).
+ */
+int m2r_scan_lanes(int codec, int n8, int n4, int64_t batch, int64_t L, int64_t H, int64_t P, int64_t G);
 
 /*
  * Stored-scale tier step (INT8/INT4/zero-carry), same row format without the

@@ -683,7 +683,7 @@ extern "C" int m2r_state_step_dense3(const void* x, const void* dt, const float*
     int wpb = 1, hpw = 1;
     const int forced = m2r_forced_step_shape();
     // several tokens: the row-split scan where it pays (16-byte pieces)
-    if (L > 1 && !forced && rows_scan_pays(MODE_DENSE3, 128, slots, (int)L) && P % 8 == 0 &&
+    if (!forced && rows_scan_lanes(MODE_DENSE3, 128, batch, (int)L, (int)H, (int)P, (int)G) > 0 &&
         (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C | (uintptr_t)y) & 15) == 0) {
       StepArgs r{};
       r.x = args.x; r.dt = args.dt; r.A = A; r.Bm = args.Bm; r.Cm = args.Cm; r.D = D; r.dt_bias = dt_bias;

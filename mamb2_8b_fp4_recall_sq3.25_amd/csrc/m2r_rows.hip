@@ -183,19 +183,50 @@ hipError_t launch_s16_rows(const S16Args& a, hipStream_t stream) {
 }
 
 // The scan pays its taking apart and putting together of the rows with the
-// first tokens.  us per call, one lane per row / this scan, at batch 1, 8 and
-// 64 (128, 1,024 and 8,192 slots):
+// first tokens.  us per call, one-lane-per-row kernel / this scan, at batch 1,
+// 8 and 64 of 128 heads of 64 rows (128, 1,024 and 8,192 slots):
 //   tier 32/32/64     8 tokens 14.4 / 11.3, 20.5 / 20.7, 102.2 / 115.7
 //                    16 tokens 24.0 / 14.8, 33.4 / 30.5, 183.1 / 180.5
 //   legacy 16/64/48   8 tokens 14.6 / 12.4, 22.2 / 23.0, 136.6 / 150.6
+//   tier 8/80/40     16 tokens at batch 8 39.9 / 41.2
 //   dense3            2 tokens 11.9 /  9.2,  4: 22.2 / 20.6, 16: 299.9 / 280.2
+//   ridge 24/44/60    8 tokens 17.9 / 23.8, 26.2 / 36.9, 145.3 / 146.2
+//                    16 tokens 30.8 / 28.2, 46.2 / 48.4, 263.8 / 227.9
+//   ridge 8/76/44    24 tokens at batch 4 and 8 52.2 / 50.9, 66.0 / 72.5
 // Wide rows over many slots (four lanes per row, see rows_lanes) come out
-// even near 64 tokens: tier 8/80/40 at batch 16, 222.0 / 221.0.
-// (A ridge scan runs where its caller brings a workspace.)
-bool rows_scan_pays(int mode, int carried, long long slots, int L) {
-  if (mode == MODE_DENSE3) return L >= (slots <= 384 ? 2 : slots <= 1024 ? 4 : 16);
-  if (slots > 1024 && carried > 72) return L >= 64;
-  return L >= (slots <= 384 ? 8 : slots <= 1024 ? 16 : 24);
+// even near 64 tokens: tier 8/80/40 at batch 16, 222.0 / 221.0; ridge 8/76/44
+// 286 / 273.
+// Between 2,048 and 3,072 slots a tier's one lane per row runs in two rounds of
+// two waves per SIMD, where the one-lane kernels hold all of them at once:
+// 32/32/64 at batch 20, 24 tokens 93.4 / 118.3, 64 tokens 234 / 277, and 24/48/56,
+// 36/24/68 and 40/16/72 lose 4 to 27% too, but 44/8/76 wins, 64 tokens 257 / 237.
+// At batch 28 32/32/64 takes 124.7 / 129.6 for 24 tokens, 163.4 / 164.3 for 32.
+// A head whose rows would leave waves of a workgroup idle (two lanes or one,
+// and heads per group that no two or four of them fill it with) stays with the
+// one-lane kernels: 8 heads in 8 groups at batch 500, 24 tokens, tier 32/32/64
+// 127 / 443.  And so does a ridge scan over more than 1,024 slots of one head per
+// group (wide rows: three), whose records serve few heads: 32 tokens of one head
+// at batch 192, 24/44/60 145 / 172, 64 of two at batch 333, 8/76/44 308 / 343.
+int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int G) {
+  const long long slots = rows_slots(B, H, P);
+  const int lanes = rows_lanes(carried, slots), rows = 64 / lanes, hpg = H / G;
+  const int blocks = rows_blocks(lanes, P), heads = rows_heads(blocks, hpg);
+  // rows a head takes room for here, and in the one-lane kernels' slots
+  const int room = 4 * rows * ((blocks * heads + 3) / 4) / heads;
+  if (L < 2 || P % 8 || room > 64 * ((P + 63) / 64)) return 0;
+  const bool wide = carried > 72;
+  int least;
+  if (mode == MODE_DENSE3) {
+    least = slots <= 384 ? 2 : slots <= 1024 ? 4 : 16;
+  } else if (mode == MODE_RIDGE) {
+    if (slots > 1024 && hpg < (wide ? 4 : 2)) return 0;
+    least = slots <= 256 ? 16 : slots <= 384 ? 20 : slots <= 1024 ? (wide && slots > 768 ? 32 : 24) : wide ? 64 : 24;
+  } else {
+    if (!wide && carried > 52 && slots > 2048 && slots <= 3072) return 0;
+    least = slots <= 384 ? 8 : slots <= 1024 ? (carried > 80 && slots > 768 ? 20 : 16) : wide ? 64
+            : slots > 3072 && slots <= 3584 ? 32 : 24;
+  }
+  return L >= least ? lanes : 0;
 }
 
 template <int N8, int N4, int NZ, int MODE>
@@ -216,3 +247,11 @@ hipError_t launch_dense3_rows(const StepArgs& a, int equalizer, hipStream_t stre
 }
 
 }  // namespace m2r
+
+using namespace m2r;
+
+extern "C" int m2r_scan_lanes(int codec, int n8, int n4, int64_t batch, int64_t L, int64_t H, int64_t P, int64_t G) {
+  if (batch <= 0 || L <= 0 || H <= 0 || P <= 0 || G <= 0 || H % G || n8 < 0 || n4 < 0) return 0;
+  if (codec < 0 || codec > 3 || (double)batch * L * H * P >= 2147483647.0) return 0;
+  return rows_scan_lanes(codec, codec == MODE_DENSE3 ? 128 : n8 + n4, batch, (int)L, (int)H, (int)P, (int)G);
+}

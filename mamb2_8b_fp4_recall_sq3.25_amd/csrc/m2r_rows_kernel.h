@@ -31,6 +31,7 @@
 // one-token step sums in the same order (the other codecs' y differ from it
 // by the order of a binary32 sum).
 #pragma once
+#include "m2r_rows.h"
 #include "m2r_step.h"
 
 namespace m2r {
@@ -728,28 +729,9 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads) {
   }
 }
 
-// Lanes per row, by the scan's 64-row slots: enough to give every SIMD a
-// wave, then fewer, as each lane repeats a token's scalar work.  us for 64
-// tokens at batch 1, 3, 4, 8, 12, 16 and 64 (128 slots each), ridge 24/44/60:
-//   8 lanes   56.3   84.0  105.6  172.5  244.4  316.9
-//   4         78.7   90.6   91.7  155.2  198.0  255.0    923
-//   2        105.8  108.8  109.7  128.9  210.2  236.0    880
-//   1        162.2  164.2  164.0  174.5  196.3  203.4    753
-// One lane has all carried coordinates and updates in registers: with more
-// than 72 they spill (8/76/44 at batch 16: 279 against 273 on four lanes).
-template <int NL>
-inline int rows_lanes(long long slots) {
-  if (slots <= 384) return 8;
-  if (slots <= 768) return 4;
-  if (slots <= 1024) return 2;
-  return slots <= 1536 || NL > 72 ? 4 : 1;
-}
-
 template <int N8, int N4, int NZ, int MODE, int LPR>
 inline hipError_t launch_rows_lanes(const StepArgs& a, int equalizer, hipStream_t stream) {
-  constexpr int RW = 64 / LPR;
-  const int blocks = (a.P + RW - 1) / RW, hpg = a.H / a.G;   // blocks of RW rows per head
-  const int heads = blocks == 1 && hpg % 4 == 0 ? 4 : blocks <= 2 && hpg % 2 == 0 ? 2 : 1;
+  const int blocks = rows_blocks(LPR, a.P), heads = rows_heads(blocks, a.H / a.G);
   const dim3 grid((unsigned)((blocks * heads + 3) / 4), (unsigned)(a.H / heads), (unsigned)a.B);
   hipLaunchKernelGGL((k_rows_scan<N8, N4, NZ, MODE, LPR>), grid, dim3(256), 0, stream, a, equalizer, heads);
   return hipGetLastError();
@@ -758,7 +740,7 @@ inline hipError_t launch_rows_lanes(const StepArgs& a, int equalizer, hipStream_
 template <int N8, int N4, int NZ, int MODE>
 inline hipError_t launch_rows_scan(const StepArgs& a, int equalizer, hipStream_t stream) {
   constexpr int NL = MODE == MODE_DENSE3 ? 128 : N8 + N4;
-  const int lanes = rows_lanes<NL>((long long)a.B * a.H * ((a.P + 63) / 64));
+  const int lanes = rows_lanes(NL, rows_slots(a.B, a.H, a.P));
   if (lanes == 8) return launch_rows_lanes<N8, N4, NZ, MODE, 8>(a, equalizer, stream);
   if (lanes == 4) return launch_rows_lanes<N8, N4, NZ, MODE, 4>(a, equalizer, stream);
   if (lanes == 2) return launch_rows_lanes<N8, N4, NZ, MODE, 2>(a, equalizer, stream);

@@ -53,11 +53,11 @@ static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   const int forced = g_forced_shape.load(std::memory_order_relaxed);
   // Several tokens: the row-split scan, where rows, inputs and readouts are
   // whole 16-byte pieces: a ridge launch that brings a workspace for its token
-  // records, another where the scan pays (m2r_rows.hip).  A forced shape keeps
+  // records, another where the scan pays (rows_scan_lanes).  A forced shape keeps
   // it away.
   const bool rows_ok = !forced && a.L > 1 && (a.dma_tiles & 1) &&
                        (((uintptr_t)a.x | (uintptr_t)a.Bm | (uintptr_t)a.Cm | (uintptr_t)a.y) & 15) == 0;
-  const bool rows = MODE == MODE_RIDGE ? a.rec != nullptr : rows_scan_pays(MODE, N8 + N4, slots, a.L);
+  const bool rows = MODE == MODE_RIDGE ? a.rec != nullptr : rows_scan_lanes(MODE, N8 + N4, a.B, a.L, a.H, a.P, a.G) > 0;
   if (rows_ok && rows)
     return launch_rows<N8, N4, NZ, MODE>(a, stream);
   if (forced == 4 * 16 && hpg % 2 == 0) {   // (4, 0): two waves per head slot

@@ -42,6 +42,7 @@ _SIGNATURES = {
     "m2r_stream_probe_phased": ([P, P, I64, I, I, I, I, I, P], I),
     "m2r_probe_butterfly": ([P, P, P], I),
     "m2r_set_step_shape": ([I, I], I),
+    "m2r_scan_lanes": ([I, I, I, I64, I64, I64, I64, I64], I),
     "m2r_causal_conv_update": ([P, I64, I64, I64, P, I64, P, P, P, I64, I64, I, I, P], I),
     "m2r_causal_conv_tokens": ([P, I64, I64, I, P, I64, I64, P, P, P, P, P, I64, I64, I64, I64, I64, I, P], I),
     "m2r_gated_rmsnorm": ([P, I64, P, I64, P, P, I64, I64, I64, I64, F32, P], I),

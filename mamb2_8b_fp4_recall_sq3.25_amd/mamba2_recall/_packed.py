@@ -59,16 +59,11 @@ def launch_packed(kind, x, dt, A, B, C, D, dt_bias, perm, tensors, *, n8, n4, nz
         if kind == "ridge":
             # a token-record workspace (results identical without) where the
             # scan that reads the records beats building each token in the
-            # step kernel; us per call, built / records, at batch 1, 8 and 64
-            # (24/44/60): 16 tokens 30.8 / 28.2, 46.2 / 48.4, 263.8 / 227.9;
-            # 8 tokens 17.9 / 23.8, 26.2 / 36.9, 145.3 / 146.2; wide rows over
-            # many slots 8/76/44 at batch 16, 64 tokens 286 / 273.  Bounded to
-            # 1 GiB beyond 1024 64-row slots.
+            # step kernel.  Bounded to 1 GiB beyond 1024 64-row slots.
             ws, ws_bytes = None, 0
-            slots = batch * heads * -(-dim // 64)
-            if length >= (16 if slots <= 384 else 24 if slots <= 1024 or n8 + n4 <= 72 else 64):
+            if length > 1 and _native.lib().m2r_scan_lanes(2, n8, n4, *geo) > 0:
                 need = int(_native.lib().m2r_ridge_records_bytes(batch, length, groups))
-                if need <= 1 << 30 or slots <= 1024:
+                if need <= 1 << 30 or batch * heads * -(-dim // 64) <= 1024:
                     ws_bytes = need
                     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
             _native.call("m2r_state_step_ridge_ws", *common, p(basis.contiguous()), p(lscale.contiguous()),

@@ -53,3 +53,33 @@ def test_step_shape_hook_accepts_documented_shapes_only():
             assert b"step shape" in lib.m2r_last_error()
     finally:
         lib.m2r_set_step_shape(0, 0)
+
+
+LEGACY, TIER, RIDGE, DENSE3 = range(4)
+
+
+def test_scan_lanes_leave_no_wave_without_rows():
+    """The multi-token scan's lanes per row: 8, 4, 2 and 1 (4 for wide rows)
+    with the slots of the 128-head model, and 0, the one-lane kernels, where a
+    workgroup's four waves would not all have rows (3 or 6 heads per group
+    with blocks of one or two waves), where a last round of waves is mostly
+    empty, for few tokens and for ragged heads."""
+    from mamba2_recall import _native
+    lanes = _native.lib().m2r_scan_lanes
+    model = (128, 64, 8)
+    for codec, n8, n4 in ((RIDGE, 24, 44), (TIER, 32, 32)):
+        assert [lanes(codec, n8, n4, b, 64, *model) for b in (1, 3, 4, 6, 7, 8, 12, 13, 16, 32, 64)] == [
+            8, 8, 4, 4, 2, 2, 4, 1, 1, 1, 1]
+        for batch, H, P, G in ((250, 8, 64, 8), (250, 8, 16, 8), (112, 8, 64, 8), (222, 9, 48, 3), (333, 6, 64, 3),
+                               (139, 9, 80, 3), (1, 65540, 48, 4)):
+            assert lanes(codec, n8, n4, batch, 64, H, P, G) == 0, (codec, batch, H, P, G)
+        assert lanes(codec, n8, n4, 300, 64, 4, 64, 1) == 4 and lanes(codec, n8, n4, 450, 64, 4, 64, 1) == 1
+        assert lanes(codec, n8, n4, 40, 64, 6, 64, 3) == 8 and lanes(codec, n8, n4, 1, 64, 8, 16, 8) == 8
+    assert [lanes(TIER, 8, 80, b, 64, *model) for b in (1, 8, 16, 64)] == [8, 2, 4, 4]
+    assert [lanes(TIER, 32, 32, b, 64, *model) for b in (17, 20, 24, 25)] == [0, 0, 0, 1]
+    assert [lanes(TIER, 32, 32, b, 24, *model) for b in (16, 28, 32, 33)] == [1, 0, 1, 1]
+    assert lanes(TIER, 44, 8, 20, 24, *model) == 1 and lanes(RIDGE, 8, 76, 333, 64, 6, 64, 3) == 0
+    assert [lanes(RIDGE, 24, 44, b, 32, 8, 64, 8) for b in (16, 100, 162)] == [8, 0, 0]
+    assert [lanes(DENSE3, 0, 0, b, 16, *model) for b in (1, 4, 8, 64)] == [8, 4, 2, 4]
+    assert [lanes(LEGACY, 16, 64, 1, L, *model) for L in (1, 2, 7, 8, 512)] == [0, 0, 0, 8, 8]
+    assert lanes(TIER, 32, 32, 1, 64, 8, 12, 8) == 0 and lanes(RIDGE, 24, 44, 1, 64, 9, 64, 2) == 0
