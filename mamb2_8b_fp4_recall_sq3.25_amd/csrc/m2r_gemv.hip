@@ -28,7 +28,9 @@
 // order through LDS, finish each output.  One activation row (the batch-1
 // decode) takes k_fp4_gemv_rows instead where it fills the chip in one
 // resident round: whole rows per wave, no barrier per row, the same sums.  Four
-// rows take k_fp4_gemv_tiles (matrix cores).
+// rows take k_fp4_gemv_tiles (matrix cores) where their outputs fill enough of
+// the chip; it sums in another order, so a row's bits are those of one or two
+// rows only below that.
 #include "m2r_device.h"
 #include "m2r_abi_util.h"
 #include "m2r_tile.h"
@@ -451,12 +453,23 @@ extern "C" int m2r_fp4_gemv_g16(const uint8_t* packed, const uint8_t* e4m3_scale
   if ((((uintptr_t)packed | (uintptr_t)u) & 15) || (u_stride % 8) || ((uintptr_t)e4m3_scales & 1))
     return m2r_fail("fp4 gemv: codes and activation rows must be 16-byte aligned, scales 2-byte aligned");
   const int kch = (int)(K / 2048);
+  int cus = 0;
   if (M == 4) {
-    int dev = 0, cus = 0;
+    int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       return m2r_fail("fp4 gemv: device query failed");
-    const dim3 grid((unsigned)std::min<int64_t>((N + 15) / 16, cus));
+  }
+  // Four rows: the matrix cores where half the CUs have a tile of 16 outputs.
+  // A workgroup loads all of the activations before its first tile and takes a
+  // whole tile's K, so with fewer tiles the dot products, which spread the
+  // outputs over every CU, are faster: us per launch, dot products / tiles, for
+  // 1,024, 1,536 and 2,048 outputs: K = 4096 4.9 / 5.9, 5.9 / 6.0, 6.8 / 6.0, K =
+  // 8192 7.0 / 10.1, 9.5 / 10.1, 11.7 / 10.1.  With K = 2048 the tiles are never
+  // slower (64 outputs 3.8 / 3.8, 1,536 4.9 / 4.0).
+  const int64_t tiles = (N + 15) / 16;
+  if (M == 4 && (kch == 1 || 2 * tiles >= cus)) {
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, cus));
 #define M2R_TILES(KK, NW, AHEAD)                                                                              \
     if (kch == KK) {                                                                                          \
       hipLaunchKernelGGL((k_fp4_gemv_tiles<KK, NW, AHEAD>), grid, dim3(64 * NW), 0, stream, packed,           \
@@ -483,6 +496,7 @@ extern "C" int m2r_fp4_gemv_g16(const uint8_t* packed, const uint8_t* e4m3_scale
   }
   M2R_GEMV(1, 1) M2R_GEMV(1, 2) M2R_GEMV(1, 4)
   M2R_GEMV(2, 1) M2R_GEMV(2, 2) M2R_GEMV(2, 4)
+  M2R_GEMV(4, 2) M2R_GEMV(4, 4)
 #undef M2R_GEMV
   return m2r_fail("fp4 gemv: supported are M in {1, 2, 4} rows of u and K in {2048, 4096, 8192}");
 }

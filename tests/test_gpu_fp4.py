@@ -275,8 +275,9 @@ def test_fp4_gemv_matches_decoded_weights(device, M, N, K):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("N,K,tiny", [(1, 4096, 1.0), (16, 8192, 1.0), (17, 2048, 1.0), (4111, 4096, 1.0),
-                                      (40003, 2048, 1.0), (5000, 8192, 2.0 ** -16)])
+@pytest.mark.parametrize("N,K,tiny", [(1, 2048, 1.0), (16, 2048, 1.0), (17, 2048, 1.0), (2033, 8192, 1.0),
+                                      (2048, 4096, 1.0), (4111, 4096, 1.0), (40003, 2048, 1.0),
+                                      (5000, 8192, 2.0 ** -16)])
 def test_fp4_gemv_four_rows_tiles(device, N, K, tiny):
     """The matrix-core GEMV (four activation rows) around its 16-row tiles and
     its batches of eight tiles per workgroup (N > 32,768), and with weights
@@ -301,6 +302,24 @@ def test_fp4_gemv_four_rows_tiles(device, N, K, tiny):
         ref = u.double() @ w.double().T
         bound = (ref.abs() * 2.0 ** -11 + (u.double().abs() @ w.double().abs().T) * K * 2.0 ** -22 + 2.0 ** -24)
         assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("N,K", [(1, 4096), (100, 8192), (1500, 4096), (2032, 8192)])
+def test_fp4_gemv_four_rows_of_few_outputs_same_bits(device, N, K):
+    """Outputs that give fewer than half the CUs a tile stay with the dot
+    products: four activation rows have the bits of two times two."""
+    from mamba2_recall import fp4
+    if torch.cuda.get_device_properties(device).multi_processor_count != 256:
+        pytest.skip("the line lies at half of 256 CUs")
+    gen = torch.Generator(device=device).manual_seed(N + K)
+    print(f"[fp4 gemv four rows, few outputs] N={N} K={K}", flush=True)
+    codes = torch.randint(0, 256, (N, K // 2), generator=gen, device=device, dtype=torch.uint8)
+    sb = torch.randint(40, 90, (N, K // 16), generator=gen, device=device, dtype=torch.uint8)
+    g = torch.full((1,), 0.003, device=device)
+    u = torch.randn((4, K), generator=gen, device=device).half()
+    four = fp4.gemv_g16(codes, sb, g, u)
+    two = torch.cat([fp4.gemv_g16(codes, sb, g, u[i:i + 2]) for i in (0, 2)])
+    assert torch.equal(four.view(torch.int16), two.view(torch.int16))
 
 
 @pytest.mark.parametrize("N,K", [(18560, 4096), (4640, 4096), (4096, 8192), (2048, 8192), (100, 2048)])
