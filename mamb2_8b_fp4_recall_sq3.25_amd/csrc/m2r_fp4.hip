@@ -313,8 +313,8 @@ __global__ __launch_bounds__(256) void k_fp4_ragged(const uint32_t* __restrict__
   report(err, flag);
 }
 
-// The same for fewer than 8 columns or other alignments: one thread per (row,
-// group).
+// The same for fewer than 8 columns, other alignments, and short G16 rows of few
+// weights (launch_unaligned): one thread per (row, group).
 template <int GROUP>
 __global__ __launch_bounds__(256) void k_fp4_padded(const uint8_t* __restrict__ packed, const void* __restrict__ scales,
                                                     const float* __restrict__ global_scale, uint16_t* __restrict__ out,
@@ -364,12 +364,18 @@ __global__ __launch_bounds__(256) void k_fp4_padded(const uint8_t* __restrict__ 
   report(err, flag);
 }
 
-// Launches the decode of a width that is not a multiple of GROUP.
+// Launches the decode of a width that is not a multiple of GROUP.  Rows of 8 to
+// 12 weights in G16 hold at most 12 stores a thread of k_fp4_padded, which is
+// then the faster until the stores fill the memory system: us, vectors /
+// padded, 2000 x 8 5.5 / 4.9, 100000 x 10 6.1 / 5.9, 100000 x 11 6.1 / 6.3, 1000000 x 8
+// 10.0 / 19.2; 13 columns 5.6 / 5.7 and 6.2 / 7.0 (2000 and 100000 rows).  In G64
+// the vectors win from 8 columns on (2000 x 8 8.6 / 10.4).
 template <int GROUP>
 static void launch_unaligned(const uint8_t* packed, const void* scales, const float* global_scale, void* out,
                             int64_t rows, int64_t cols, uint32_t* flag, hipStream_t stream) {
   const int64_t blocks = (rows * cols + 8191) / 8192;
-  if (cols >= 8 && cols < (1 << 30) && blocks <= 0x7FFFFFFF && ((uintptr_t)packed & 3) == 0 &&
+  const bool small = GROUP == 16 && cols <= 12 && rows * cols <= 1 << 20;
+  if (cols >= 8 && !small && cols < (1 << 30) && blocks <= 0x7FFFFFFF && ((uintptr_t)packed & 3) == 0 &&
       ((uintptr_t)out & 15) == 0) {
     hipLaunchKernelGGL((k_fp4_ragged<GROUP>), dim3((unsigned)blocks), dim3(256), 0, stream, (const uint32_t*)packed,
                        scales, global_scale, (uint16_t*)out, rows, cols, flag);

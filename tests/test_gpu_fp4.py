@@ -176,11 +176,13 @@ def test_g64_random_bit_exact(oracle, device, rows, cols):
 
 @pytest.mark.parametrize("group", [16, 64])
 @pytest.mark.parametrize("rows,cols", [(3, 8), (5, 9), (2, 15), (7, 17), (67, 31), (1000, 33), (129, 63), (5, 65),
-                                       (3, 2730), (3, 2731), (9, 4100), (2, 8191), (3, 8193), (1, 20001), (4, 7)])
+                                       (3, 2730), (3, 2731), (9, 4100), (2, 8191), (3, 8193), (1, 20001), (4, 7),
+                                       (131080, 8), (120001, 9), (87400, 12)])
 def test_ragged_widths_bit_exact(oracle, device, group, rows, cols):
     """Widths that are no multiple of the group: rows and groups that end
     anywhere in an eight-weight vector, a partial last vector, widths on both
-    sides of a workgroup's 8192 weights, and one below eight columns."""
+    sides of a workgroup's 8192 weights, one below eight columns, and short
+    rows on both sides of 2^20 weights."""
     if cols % group == 0:
         return
     rng = np.random.default_rng(rows * 31 + cols + group)
