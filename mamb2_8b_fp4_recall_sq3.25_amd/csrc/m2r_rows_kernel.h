@@ -561,9 +561,11 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads) {
       bool unclamped = finite_in, zero[SETS];
 #pragma unroll
       for (int e = 0; e < SETS; ++e) {
-        // a stored scale that is zero (underflowed) or infinite: code 0
-        zero[e] = !DEN32 && (!(stored[e] > 0.f) || stored[e] == __builtin_inff());
-        unclamped = unclamped && (DEN32 || zero[e] || stored[e] >= 0x1p-14f);
+        zero[e] = !DEN32 && stored[e] == 0.f;
+        // (2^-14 to 65504, as one comparison of integers; an overflowed scale
+        // has no reciprocal for the two-sided quantizer)
+        const bool normal = __builtin_bit_cast(uint32_t, stored[e]) - 0x38800000u <= 0x477FE000u - 0x38800000u;
+        unclamped = unclamped && (DEN32 || zero[e] || normal);
       }
       if (__builtin_amdgcn_ballot_w64(!unclamped) == 0) {
         float yh[SETS], yl[SETS];
@@ -606,8 +608,8 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads) {
           });
         }
       } else {
-        // not finite, or a binary16-subnormal stored scale: clamped exact
-        // quotients (a zero, infinite or NaN divisor divides through d = 1, y = 0)
+        // not finite, or a binary16-subnormal or infinite stored scale: clamped
+        // exact quotients (a zero, infinite or NaN divisor divides through d = 1, y = 0)
         float d[SETS], ry[SETS], top[SETS];
 #pragma unroll
         for (int e = 0; e < SETS; ++e) {
