@@ -204,9 +204,11 @@ hipError_t launch_s16_rows(const S16Args& a, hipStream_t stream) {
 // A head whose rows would leave waves of a workgroup idle (two lanes or one,
 // and heads per group that no two or four of them fill it with) stays with the
 // one-lane kernels: 8 heads in 8 groups at batch 500, 24 tokens, tier 32/32/64
-// 127 / 443.  And so does a ridge scan over more than 1,024 slots of one head per
-// group (wide rows: three), whose records serve few heads: 32 tokens of one head
-// at batch 192, 24/44/60 145 / 172, 64 of two at batch 333, 8/76/44 308 / 343.
+// 127 / 443.  A ridge scan's records serve the heads of a group: one head per
+// group pays from 64 tokens on to 1,280 slots (batch 138: 32 tokens 141 / 144, 64
+// 273 / 255), and not above (batch 175, 128 tokens 535 / 566); wide rows of two or
+// three heads to 1,536 (batch 122 of 9 heads, 64 tokens 294 / 214; batch 333 of 6,
+// 308 / 343).
 int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int G) {
   const long long slots = rows_slots(B, H, P);
   const int lanes = rows_lanes(carried, slots), rows = 64 / lanes, hpg = H / G;
@@ -219,8 +221,8 @@ int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int
   if (mode == MODE_DENSE3) {
     least = slots <= 384 ? 2 : slots <= 1024 ? 4 : 16;
   } else if (mode == MODE_RIDGE) {
-    if (slots > 1024 && hpg < (wide ? 4 : 2)) return 0;
-    least = slots <= 256 ? 16 : slots <= 384 ? 20 : slots <= 1024 ? (wide && slots > 768 ? 32 : 24) : wide ? 64 : 24;
+    if (slots > (hpg == 1 ? 1280 : 1536) && hpg < (wide ? 4 : 2)) return 0;
+    least = slots > 1024 && hpg == 1 ? 64 : slots <= 256 ? 16 : slots <= 384 ? 20 : slots <= 1024 ? (wide && slots > 768 ? 32 : 24) : wide ? 64 : 24;
   } else {
     if (!wide && carried > 52 && slots > 2048 && slots <= 3072) return 0;
     least = slots <= 384 ? 8 : slots <= 1024 ? (carried > 80 && slots > 768 ? 20 : 16) : wide ? 64
