@@ -72,7 +72,9 @@ int m2r_state_step_ridge_ws(const void* x, const void* dt, const float* A, const
                             uint8_t* q4, uint8_t* latent, void* s8, void* s4, void* y, int64_t batch, int64_t L,
                             int64_t H, int64_t P, int64_t G, int n8, int n4, int nz, void* workspace,
                             int64_t workspace_bytes, hipStream_t stream);
-/* Workspace bytes of m2r_state_step_ridge_ws: batch * L * G records of 1 KiB. */
+/* Workspace bytes of m2r_state_step_ridge_ws: batch * G records of 1 KiB for each
+ * of min(L, piece) tokens; longer calls run in pieces, of as many tokens as fit
+ * 256 MiB (a multiple of 64, at least 64). */
 int64_t m2r_ridge_records_bytes(int64_t batch, int64_t L, int64_t G);
 /*
  * Lanes per row (8, 4, 2 or 1) of the multi-token scan where it beats the

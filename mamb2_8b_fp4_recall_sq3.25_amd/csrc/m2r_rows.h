@@ -56,6 +56,15 @@ int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int
 template <int N8, int N4, int NZ, int MODE>
 hipError_t launch_rows(const StepArgs& a, hipStream_t stream);
 
+// Tokens whose records a ridge scan holds at a time: those of 256 MiB, in
+// whole dt batches of 64.  A piece costs a trip of the carry through memory and
+// two launches: with 128 MiB the second half of 256 tokens at batch 128 took
+// 1.3% (24/44/60 5,537 -> 5,608 us), the last 32 of 96 at batch 256 4 to 5%.
+inline int64_t ridge_piece(int64_t batch, int64_t G) {
+  const int64_t tokens = (256 << 10) / (batch * G);
+  return tokens < 64 ? 64 : tokens & ~(int64_t)63;
+}
+
 // The same scan of dense 3-bit rows: a.lo the codes, a.s8 the scale pairs,
 // a.perm the table.  P % 8 == 0; every array 16-byte aligned.
 hipError_t launch_dense3_rows(const StepArgs& a, int equalizer, hipStream_t stream);

@@ -1,15 +1,23 @@
 // The row-split multi-token scan of ridge-latent rows (m2r_rows_kernel.h),
-// behind the kernel that writes its token records.
+// behind the kernel that writes its token records, a piece of the tokens at a
+// time: the codes between pieces are the ones between tokens.
 #include "m2r_rows_kernel.h"
 #include "m2r_rows.h"
+
+#include <algorithm>
 
 namespace m2r {
 
 template <int N8, int N4, int NZ, int MODE>
 hipError_t launch_rows(const StepArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((k_token_records<N8, N4, NZ>), dim3((a.L + REC_TOKENS - 1) / REC_TOKENS, a.G, a.B), dim3(256), 0,
-                     stream, a, (float*)a.rec);
-  return launch_rows_scan<N8, N4, NZ, MODE>(a, 0, stream);
+  const int piece = (int)ridge_piece(a.B, a.G);
+  for (int first = 0; first < a.L; first += piece) {
+    const int tokens = std::min(piece, a.L - first);
+    hipLaunchKernelGGL((k_token_records<N8, N4, NZ>), dim3((tokens + REC_TOKENS - 1) / REC_TOKENS, a.G, a.B), dim3(256),
+                       0, stream, a, (float*)a.rec, first, tokens);
+    if (hipError_t e = launch_rows_scan<N8, N4, NZ, MODE>(a, 0, first, tokens, stream)) return e;
+  }
+  return hipSuccess;
 }
 template hipError_t launch_rows<36, 20, 72, MODE_RIDGE>(const StepArgs&, hipStream_t);
 template hipError_t launch_rows<16, 60, 52, MODE_RIDGE>(const StepArgs&, hipStream_t);

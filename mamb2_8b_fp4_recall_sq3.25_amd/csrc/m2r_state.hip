@@ -3,6 +3,7 @@
 #include "m2r_abi_util.h"
 #include "m2r_rows.h"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <initializer_list>
@@ -41,8 +42,8 @@ static void launch_shape(const StepArgs& a, dim3 grid, hipStream_t stream) {
   }
 }
 
-// args.rec: a token-record workspace of at least B * L * G records (or
-// null), for the row-split scan of a multi-token ridge launch.
+// args.rec: a token-record workspace (m2r_ridge_records_bytes, or null), for
+// the row-split scan of a multi-token ridge launch.
 template <int N8, int N4, int NZ, int MODE>
 static hipError_t launch_layout(const StepArgs& args, hipStream_t stream) {
   StepArgs a = args;
@@ -163,7 +164,7 @@ static int check_geometry(int64_t batch, int64_t L, int64_t H, int64_t P, int64_
 
 extern "C" int64_t m2r_ridge_records_bytes(int64_t batch, int64_t L, int64_t G) {
   if (batch <= 0 || L <= 0 || G <= 0) return 0;
-  return batch * L * G * (int64_t)(REC_FLOATS * sizeof(float));
+  return batch * std::min(L, ridge_piece(batch, G)) * G * (int64_t)(REC_FLOATS * sizeof(float));
 }
 
 extern "C" int m2r_state_step_ridge_ws(const void* x, const void* dt, const float* A, const void* B, const void* C,

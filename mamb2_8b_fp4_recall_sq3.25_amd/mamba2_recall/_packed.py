@@ -59,13 +59,11 @@ def launch_packed(kind, x, dt, A, B, C, D, dt_bias, perm, tensors, *, n8, n4, nz
         if kind == "ridge":
             # a token-record workspace (results identical without) where the
             # scan that reads the records beats building each token in the
-            # step kernel.  Bounded to 1 GiB beyond 1024 64-row slots.
+            # step kernel
             ws, ws_bytes = None, 0
             if length > 1 and _native.lib().m2r_scan_lanes(2, n8, n4, *geo) > 0:
-                need = int(_native.lib().m2r_ridge_records_bytes(batch, length, groups))
-                if need <= 1 << 30 or batch * heads * -(-dim // 64) <= 1024:
-                    ws_bytes = need
-                    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
+                ws_bytes = int(_native.lib().m2r_ridge_records_bytes(batch, length, groups))
+                ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
             _native.call("m2r_state_step_ridge_ws", *common, p(basis.contiguous()), p(lscale.contiguous()),
                          p(pred.contiguous()), p(tensors["lo"]), p(tensors["hi"]), p(tensors["q4"]),
                          p(tensors["latent"]), p(tensors["s8"]), p(tensors["s4"]), p(y), *geo, n8, n4, nz,

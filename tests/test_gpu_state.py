@@ -409,6 +409,36 @@ def test_ridge_workspace_same_bits_as_without(device, layout, batch, H, G):
         assert differ == 0, f"{k}: {differ} of {out[0][k].numel()} differ"
 
 
+@pytest.mark.parametrize("layout,batch,L", [("24_48_56", 512, 150), ("8_80_40", 600, 129)])
+def test_ridge_records_in_pieces(device, layout, batch, L):
+    """Calls whose token records exceed the workspace run in pieces of 64
+    tokens (the last one partial): the results of the call without a
+    workspace, and nothing written past it."""
+    from mamba2_recall import _native, ridge_codec
+    n8, n4, nz = ridge_counts(layout)
+    H, P, G = 16, 16, 8
+    print(f"[ridge pieces] layout={layout} B={batch} L={L}", flush=True)
+    rng = np.random.default_rng(L)
+    inp = cases.step_inputs(rng, batch, L, H, P, G)
+    sta = cases.ridge_statics(rng, G, n8, n4, nz)
+    st0 = cases.random_packed_state(rng, batch, H, P, n8, n4, latent=True)
+    t = device_inputs(inp, device)
+    perm = torch.from_numpy(inp["perm"]).to(device)
+    basis, ls, pred = (dev16(sta[k], device) for k in ("basis", "lscale", "pred"))
+    need = int(_native.lib().m2r_ridge_records_bytes(batch, L, G))
+    assert need == batch * 64 * G * 1024
+    whole = torch.full((need // 4 + 1024,), float("nan"), dtype=torch.float32, device=device)
+    out = []
+    for ws in (None, whole[:need // 4]):
+        state = ridge_codec.allocate_state(batch, H, P, 128, device, layout=layout)
+        to_state(st0, state, device)
+        y = _ridge_step_direct(t, perm, basis, ls, pred, state, layout, ws)
+        out.append(dict({k: v.view(torch.uint8) for k, v in state.tensors.items()}, y=y.view(torch.int16)))
+    for k in out[0]:
+        assert torch.equal(out[0][k], out[1][k]), k
+    assert bool(torch.isnan(whole[need // 4:]).all()) and not bool(torch.isnan(whole[:need // 4]).any())
+
+
 def test_ridge_token_records_graph_replays_match_eager(device):
     """The records kernel and the record-fed step captured in a HIP graph
     (one workspace, static inputs): three replays, each from the same

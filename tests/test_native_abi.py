@@ -84,3 +84,16 @@ def test_scan_lanes_leave_no_wave_without_rows():
     assert [lanes(DENSE3, 0, 0, b, 16, *model) for b in (1, 4, 8, 64)] == [8, 4, 2, 4]
     assert [lanes(LEGACY, 16, 64, 1, L, *model) for L in (1, 2, 7, 8, 512)] == [0, 0, 0, 8, 8]
     assert lanes(TIER, 32, 32, 1, 64, 8, 12, 8) == 0 and lanes(RIDGE, 24, 44, 1, 64, 9, 64, 2) == 0
+
+
+def test_ridge_workspace_is_bounded():
+    """1 KiB per batch row, token and group up to 256 MiB, then the records of
+    a piece of the tokens, at least 64: no more than about the packed state of
+    8 heads of 128 rows per group."""
+    from mamba2_recall import _native
+    need = _native.lib().m2r_ridge_records_bytes
+    assert need(1, 512, 8) == 512 * 8 << 10 and need(3, 19, 8) == 3 * 19 * 8 << 10
+    assert need(64, 512, 8) == need(64, 100000, 8) == 256 << 20
+    assert need(60, 100000, 8) == 60 * 512 * 8 << 10
+    assert need(4096, 64, 8) == need(4096, 1000, 8) == 4096 * 64 * 8 << 10
+    assert need(0, 5, 8) == 0
