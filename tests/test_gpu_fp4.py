@@ -283,8 +283,11 @@ def test_fp4_gemv_matches_decoded_weights(device, M, N, K):
 def test_fp4_gemv_four_rows_tiles(device, N, K, tiny):
     """The matrix-core GEMV (four activation rows) around its 16-row tiles and
     its batches of eight tiles per workgroup (N > 32,768), and with weights
-    down to binary16 subnormals, against float64 within the bound of the test
-    above: products of binary16 values are exact in binary32."""
+    down to binary16 subnormals, against float64 within the bounds of the test
+    above: products of binary16 values are exact in binary32.  Then with
+    weights that are multiples of 1/2 up to 24 and whole activations up to 8:
+    every sum is exact in binary32 (below 2^23 halves), so the outputs must
+    equal the product, and a lost or misplaced code word shows."""
     from mamba2_recall import fp4
     gen = torch.Generator(device=device).manual_seed(N + K)
     print(f"[fp4 gemv tiles] N={N} K={K} tiny={tiny}", flush=True)
@@ -302,8 +305,16 @@ def test_fp4_gemv_four_rows_tiles(device, N, K, tiny):
     for u in (wide[:, :K].contiguous(), wide[:, :K]):   # the second with a row stride of its own
         y = fp4.gemv_g16(codes, sb, g, u)
         ref = u.double() @ w.double().T
+        assert float((y.double() - ref).norm() / ref.norm()) <= (1e-3 if tiny == 1.0 else 1e-2)   # (subnormal outputs)
         bound = (ref.abs() * 2.0 ** -11 + (u.double().abs() @ w.double().abs().T) * K * 2.0 ** -22 + 2.0 ** -24)
         assert bool(((y.double() - ref).abs() <= bound).all())
+    whole = torch.tensor([0x38, 0x40, 0x48], device=device, dtype=torch.uint8)   # block scales 1, 2 and 4
+    sb = whole[torch.randint(0, 3, (N, K // 16), generator=gen, device=device)]
+    one = torch.ones(1, device=device)
+    w = fp4.decode_packet(dict(format="fp4_g16_e4m3", shape=[N, K], group_size=16, packed=codes,
+                               scales=sb.view(torch.float8_e4m3fn), global_scale=one.reshape(())))
+    u = torch.randint(-8, 9, (4, K), generator=gen, device=device).half()
+    assert torch.equal(fp4.gemv_g16(codes, sb, one, u), (u.double() @ w.double().T).half())
 
 
 @pytest.mark.parametrize("N,K", [(1, 4096), (100, 8192), (1500, 4096), (2032, 8192)])

@@ -186,6 +186,30 @@ def test_conv_tokens_bit_exact(device, sizes, batch, tokens, history, with_bias,
         assert bool(same.all()), f"{int((~same).sum())} outputs differ"
 
 
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("tokens", [1, 7, 37, 1024])
+@pytest.mark.parametrize("history", [False, True])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_conv_tokens_equals_the_modules(device, batch, tokens, history, with_bias):
+    """At the model's 10,240 channels, the bits of the modules it stands in
+    for: act(conv(series)) over the history and the new inputs."""
+    from mamba2_recall.state_quant import conv_tokens
+    sizes = (8192, 1024, 1024)
+    channels = sum(sizes)
+    gen = torch.Generator(device=device).manual_seed(31 * tokens + batch)
+    print(f"[conv tokens modules] B={batch} L={tokens} history={history} bias={with_bias}", flush=True)
+    conv, act = conv_modules(sizes, with_bias, device, gen), nn.SiLU()
+    win = make_window(batch, channels, "time_major", device, gen, 1.0)
+    value = torch.randn(batch, tokens, channels + 136, generator=gen, device=device).half()[..., 64:64 + channels]
+    lead = 3 if history else 0
+    with torch.no_grad():
+        series = torch.cat((win[:, :, 4 - lead:], value.transpose(1, 2)), dim=-1)
+        want = act(conv(series).transpose(1, 2)[:, :lead + tokens])[:, lead:]
+    got = torch.cat(conv_tokens(win, value, conv.weight, conv.bias, sizes, history=history), dim=-1)
+    differ = int((got.view(torch.int16) != want.contiguous().view(torch.int16)).sum())
+    assert differ == 0, f"{differ} of {got.numel()} outputs differ"
+
+
 def test_conv_tokens_leaves_other_modules_alone(device):
     from mamba2_recall.state_quant import conv_tokens_supported
     gen = torch.Generator(device=device).manual_seed(3)
