@@ -233,7 +233,7 @@ int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int
 
 template <int N8, int N4, int NZ, int MODE>
 hipError_t launch_rows(const StepArgs& a, hipStream_t stream) {
-  return launch_rows_scan<N8, N4, NZ, MODE>(a, 0, 0, a.L, stream);
+  return launch_rows_scan<N8, N4, NZ, MODE>(a, 0, a.L, stream);
 }
 template hipError_t launch_rows<16, 64, 48, MODE_LEGACY>(const StepArgs&, hipStream_t);
 template hipError_t launch_rows<16, 64, 48, MODE_STORED>(const StepArgs&, hipStream_t);
@@ -245,7 +245,7 @@ template hipError_t launch_rows<40, 16, 72, MODE_STORED>(const StepArgs&, hipStr
 template hipError_t launch_rows<44, 8, 76, MODE_STORED>(const StepArgs&, hipStream_t);
 
 hipError_t launch_dense3_rows(const StepArgs& a, int equalizer, hipStream_t stream) {
-  return launch_rows_scan<64, 64, 0, MODE_DENSE3>(a, equalizer, 0, a.L, stream);
+  return launch_rows_scan<64, 64, 0, MODE_DENSE3>(a, equalizer, a.L, stream);
 }
 
 }  // namespace m2r

@@ -155,7 +155,7 @@ __device__ __forceinline__ float recip_near(float d) {
 
 template <int N8, int N4, int NZ, int MODE, int LPR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LPR == 8 || LPR == 4 ? 3 : 2, 8)))
-void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int tokens) {
+void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int tokens) {
   using Geo = RowGeom<N8, N4, MODE, LPR>;
   using Smem = RowsSmem<N8, N4, MODE, LPR>;
   constexpr bool RIDGE = MODE == MODE_RIDGE, D3 = MODE == MODE_DENSE3, DEN32 = MODE == MODE_LEGACY || D3;
@@ -168,9 +168,8 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int t
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.z;
-  // tokens first_token .. + L of the call (a ridge scan's records: these alone)
+  // the first L of a batch row's a.L tokens (a ridge scan's records: these alone)
   const int H = a.H, P = a.P, G = a.G, L = RIDGE ? tokens : a.L;
-  const int bt0 = b * a.L + (RIDGE ? first_token : 0);
   // a wave's rows: RW consecutive p of one head; the four waves take
   // consecutive blocks of wg_heads heads of one group
   const int wave_blocks = 4 / wg_heads;
@@ -234,7 +233,7 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int t
   // x and y: piece i of 8 rows of a token, tid + 256 k over (token, piece)
   auto xy_row = [&](int i, int t, size_t& at) {   // false: past P
     const int w = i / (RW / 8), p = p_of(w) + 8 * (i % (RW / 8));
-    at = ((size_t)(bt0 + t) * H + head_of(w)) * P + p;
+    at = ((size_t)(b * a.L + t) * H + head_of(w)) * P + p;
     return p < P;
   };
   auto load_block = [&](int t0) {   // (past the last token: stale values, never stepped)
@@ -242,13 +241,13 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int t
 #pragma unroll
       for (int k = 0; k < PIECES; ++k) {
         const int t = t0 + wave + 4 * k;
-        if (t < L) piece[k] = ((const u32x4*)(a.rec + ((size_t)b * L + t) * G * REC_FLOATS + g * REC_FLOATS))[lane];
+        if (t < L) piece[k] = ((const u32x4*)(a.rec + ((size_t)(b * L + t) * G + g) * REC_FLOATS))[lane];
       }
     } else {
 #pragma unroll
       for (int k = 0; k < PIECES; ++k) {
         const int t = t0 + rt + 8 * k;
-        if (t < L) piece[k] = *(const u32x4*)(raw_src + ((size_t)(bt0 + t) * G + g) * 128);
+        if (t < L) piece[k] = *(const u32x4*)(raw_src + ((size_t)(b * a.L + t) * G + g) * 128);
       }
     }
 #pragma unroll
@@ -410,7 +409,7 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int t
     // workgroup's waves take turns, else each wave does its own head's
     if ((t0 & 63) == 0 && (wg_heads > 1 || wave == ((t0 >> 6) & 3))) {
       const int t = min(t0 + lane, L - 1);
-      const float2 v = dt_activation<false>(h2f(a.dt[(size_t)(bt0 + t) * H + h]) + bias, av);
+      const float2 v = dt_activation<false>(h2f(a.dt[(size_t)(b * a.L + t) * H + h]) + bias, av);
       // |b| < 2^30 (2^16 without an equalizer), |dt| < 2^60 and |decay| <
       // 2^100 keep every update of finite operands finite
       const bool bounded = __builtin_fabsf(v.x) < 0x1p60f && __builtin_fabsf(v.y) < 0x1p100f;
@@ -734,22 +733,22 @@ void k_rows_scan(StepArgs a, int equalizer, int wg_heads, int first_token, int t
 }
 
 template <int N8, int N4, int NZ, int MODE, int LPR>
-inline hipError_t launch_rows_lanes(const StepArgs& a, int equalizer, int first_token, int tokens, hipStream_t stream) {
+inline hipError_t launch_rows_lanes(const StepArgs& a, int equalizer, int tokens, hipStream_t stream) {
   const int blocks = rows_blocks(LPR, a.P), heads = rows_heads(blocks, a.H / a.G);
   const dim3 grid((unsigned)((blocks * heads + 3) / 4), (unsigned)(a.H / heads), (unsigned)a.B);
   hipLaunchKernelGGL((k_rows_scan<N8, N4, NZ, MODE, LPR>), grid, dim3(256), 0, stream, a, equalizer, heads,
-                     first_token, tokens);
+                     tokens);
   return hipGetLastError();
 }
 
 template <int N8, int N4, int NZ, int MODE>
-inline hipError_t launch_rows_scan(const StepArgs& a, int equalizer, int first_token, int tokens, hipStream_t stream) {
+inline hipError_t launch_rows_scan(const StepArgs& a, int equalizer, int tokens, hipStream_t stream) {
   constexpr int NL = MODE == MODE_DENSE3 ? 128 : N8 + N4;
   const int lanes = rows_lanes(NL, rows_slots(a.B, a.H, a.P));
-  if (lanes == 8) return launch_rows_lanes<N8, N4, NZ, MODE, 8>(a, equalizer, first_token, tokens, stream);
-  if (lanes == 4) return launch_rows_lanes<N8, N4, NZ, MODE, 4>(a, equalizer, first_token, tokens, stream);
-  if (lanes == 2) return launch_rows_lanes<N8, N4, NZ, MODE, 2>(a, equalizer, first_token, tokens, stream);
-  if constexpr (NL <= 72) return launch_rows_lanes<N8, N4, NZ, MODE, 1>(a, equalizer, first_token, tokens, stream);
+  if (lanes == 8) return launch_rows_lanes<N8, N4, NZ, MODE, 8>(a, equalizer, tokens, stream);
+  if (lanes == 4) return launch_rows_lanes<N8, N4, NZ, MODE, 4>(a, equalizer, tokens, stream);
+  if (lanes == 2) return launch_rows_lanes<N8, N4, NZ, MODE, 2>(a, equalizer, tokens, stream);
+  if constexpr (NL <= 72) return launch_rows_lanes<N8, N4, NZ, MODE, 1>(a, equalizer, tokens, stream);
   return hipErrorInvalidValue;   // (rows_lanes never asks for one lane there)
 }
 

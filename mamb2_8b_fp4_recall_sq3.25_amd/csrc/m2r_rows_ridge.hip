@@ -13,9 +13,15 @@ hipError_t launch_rows(const StepArgs& a, hipStream_t stream) {
   const int piece = (int)ridge_piece(a.B, a.G);
   for (int first = 0; first < a.L; first += piece) {
     const int tokens = std::min(piece, a.L - first);
+    StepArgs p = a;   // its tokens are the first of each batch row from these pointers on
+    p.x += (size_t)first * a.H * a.P;
+    p.y += (size_t)first * a.H * a.P;
+    p.dt += (size_t)first * a.H;
+    p.Bm += (size_t)first * a.G * 128;
+    p.Cm += (size_t)first * a.G * 128;
     hipLaunchKernelGGL((k_token_records<N8, N4, NZ>), dim3((tokens + REC_TOKENS - 1) / REC_TOKENS, a.G, a.B), dim3(256),
-                       0, stream, a, (float*)a.rec, first, tokens);
-    if (hipError_t e = launch_rows_scan<N8, N4, NZ, MODE>(a, 0, first, tokens, stream)) return e;
+                       0, stream, p, (float*)a.rec, tokens);
+    if (hipError_t e = launch_rows_scan<N8, N4, NZ, MODE>(p, 0, tokens, stream)) return e;
   }
   return hipSuccess;
 }

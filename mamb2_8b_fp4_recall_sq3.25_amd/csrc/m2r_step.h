@@ -1693,8 +1693,8 @@ void k_state_step(StepArgs a) {
 // batch row) runs the split token build of every token (wave_token_build with
 // four waves: the same gathers, sums, ridge correction and dead-tier trees,
 // so the same bits) and wave 0 stores the state-independent values as the
-// token's record, those of tokens first .. first + count of the call at
-// rec[((b count + t - first) G + g) REC_FLOATS].  Each token's inputs
+// token's record, those of the first `count` of a batch row's L tokens at
+// rec[((b count + t) G + g) REC_FLOATS].  Each token's inputs
 // are loaded while the previous token is built.  Needs 16-byte
 // aligned predictor and 4-byte aligned B and C (StepArgs::dma_tiles bit 0).
 constexpr int REC_TOKENS = 8;
@@ -1709,7 +1709,7 @@ struct RecordSmem {
 };
 
 template <int N8, int N4, int NZ>
-__global__ __launch_bounds__(256) void k_token_records(StepArgs a, float* rec, int first, int count) {
+__global__ __launch_bounds__(256) void k_token_records(StepArgs a, float* rec, int count) {
   constexpr int NL = N8 + N4, F = NL + 2, RZ = next_pow2(NZ);
   using Smem = RecordSmem<N8, N4, NZ>;
   constexpr int PRED_OPS16 = (Smem::PRED_DW + 255) / 256;
@@ -1718,7 +1718,7 @@ __global__ __launch_bounds__(256) void k_token_records(StepArgs a, float* rec, i
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.y, b = blockIdx.z;
-  const int L = a.L, t0 = first + blockIdx.x * REC_TOKENS, t1 = min(t0 + REC_TOKENS, first + count);
+  const int L = a.L, t0 = blockIdx.x * REC_TOKENS, t1 = min(t0 + REC_TOKENS, count);
   const int h0 = g * (a.H / a.G);   // a head of the group (the build also copies x of its rows: unused)
   // the group's predictor (16-byte chunks; lanes past the end re-read the
   // last one), permutation and dead-tier basis, as the step kernel loads them
@@ -1766,7 +1766,7 @@ __global__ __launch_bounds__(256) void k_token_records(StepArgs a, float* rec, i
         else if (idx >= REC_B && idx < REC_B + NL) x = bv;
         v[i] = x;
       }
-      float4* dst = (float4*)(rec + (((size_t)b * count + t - first) * a.G + g) * REC_FLOATS);
+      float4* dst = (float4*)(rec + ((size_t)(b * count + t) * a.G + g) * REC_FLOATS);
       dst[lane] = make_float4(v[0], v[1], v[2], v[3]);
     }
   }
