@@ -159,10 +159,10 @@ constexpr int tier_packed_of(int j, int T) {
 // INT8 tier is never split between two waves); the other two are the valid
 // cuts that make the largest segment smallest, then the sum of the segments'
 // squares (the lowest cuts on a further tie).  Each
-// segment's readout is one fma chain per half (half_pos), summed, and the row's
-// readout the segments' left fold ((s0 + s1) + s2) + s3, on every workgroup shape
-// and in the multi-token scan, so that y does not depend on how tokens are
-// split over calls or on the batch.  A slot stepped by four
+// segment's readout is one fma chain per tier (ridge: per half, half_pos, the
+// order of its multi-token scan), summed, and the row's readout the segments'
+// left fold ((s0 + s1) + s2) + s3 on every
+// workgroup shape.  A slot stepped by four
 // waves gives wave r segment r; by two waves, wave 0 the segments before the
 // two-wave split and wave 1 the others.
 constexpr bool seg_cut_ok(int n8, int p) { return p <= n8 ? (p % 8 == 0 || p == n8) : (p - n8) % 8 == 0; }
@@ -227,6 +227,14 @@ __host__ __device__ __forceinline__ constexpr int half_of(int p) {
                 S4 = half_pos(N8, N4, 4), S5 = half_pos(N8, N4, 5), S6 = half_pos(N8, N4, 6),
                 S7 = half_pos(N8, N4, 7);
   return p < S4 ? (p < S2 ? (p < S1 ? 0 : 1) : (p < S3 ? 2 : 3)) : (p < S6 ? (p < S5 ? 4 : 5) : (p < S7 ? 6 : 7));
+}
+// readout chain of p: its half, or (MODE other than ridge: one chain per
+// segment and tier) the first half of its segment in its tier
+template <int N8, int N4, int MODE>
+__host__ __device__ __forceinline__ constexpr int chain_of(int p) {
+  const int h = half_of<N8, N4>(p), s = h & ~1;
+  constexpr int HB = half_of<N8, N4>(N8);   // the INT4 tier's first half
+  return MODE == MODE_RIDGE || (s < HB && h >= HB) ? h : s;
 }
 // bit r: wave r of a WPS-wave slot steps INT8 (TIER4 false) or INT4 coordinates
 template <int N8, int N4, int WPS, bool TIER4>
@@ -639,7 +647,7 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
 // IEEE product for infinite and NaN scales (where the fused form gives
 // inf - inf).
 //
-// Readout: rs[hf] is set, for each half hf (half_of) in the tier's
+// Readout: rs[hf] is set, for each chain hf (chain_of) in the tier's
 // coordinates, to the binary32 chain of prior * w over them (w the readout
 // weights; one chain is live at a time, chains being contiguous runs of
 // chunks).  `bdt4` and `cw4` are the head's B*dt and the
@@ -649,7 +657,7 @@ __device__ __forceinline__ void wave_token_build(WaveToken<N8, N4, HPW>& wt, Gro
 // maximum of |update|), tier_requant the second (the new scale and codes
 // from the maximum over the whole tier): a tier split between waves runs the
 // halves on its parts with the parts' maxima combined in between.
-template <int N, bool INT8, bool EXACT, int N8, int N4, int P0>
+template <int N, bool INT8, bool EXACT, int N8, int N4, int P0, int MODE>
 __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float decay, float x, const f32x4* bdt4,
                                              const f32x4* cw4, float (&rs)[8], float (&v)[N]) {
   constexpr float BIAS = INT8 ? 128.0f : 8.0f;
@@ -677,7 +685,7 @@ __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float 
     asm volatile("" : "+v"(cc));
     const uint32_t h01 = __builtin_amdgcn_perm(0x64646464u, cc, 0x04010400u);
     const uint32_t h23 = __builtin_amdgcn_perm(0x64646464u, cc, 0x04030402u);
-    const int hf = half_of<N8, N4>(P0 + i0);   // a whole chunk lies in one chain
+    const int hf = chain_of<N8, N4, MODE>(P0 + i0);   // a whole chunk lies in one chain
     float pr[4];
     if constexpr (EXACT) {
       const f16x2 q01 = pk_add_h(__builtin_bit_cast(f16x2, h01), nbias);
@@ -698,7 +706,7 @@ __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float 
     }
     amax = max3_abs(amax, v[i0], v[i0 + 1]);
     amax = max3_abs(amax, v[i0 + 2], v[i0 + 3]);
-    if (i0 + 4 == N || half_of<N8, N4>(P0 + i0 + 4) != hf) {   // the chain's last chunk
+    if (i0 + 4 == N || chain_of<N8, N4, MODE>(P0 + i0 + 4) != hf) {   // the chain's last chunk
       rs[hf] = racc;
       racc = 0.f;
     }
@@ -708,18 +716,18 @@ __device__ __forceinline__ float tier_update(const uint32_t* c, float sc, float 
   // requantization, which keeps every prior and LDS operand live at once.
 #pragma unroll
   for (int i0 = 0; i0 < N; i0 += 4) {
-    const int hf = half_of<N8, N4>(P0 + i0);
-    if (i0 + 4 == N || half_of<N8, N4>(P0 + i0 + 4) != hf) asm volatile("" : "+v"(rs[hf]));
+    const int hf = chain_of<N8, N4, MODE>(P0 + i0);
+    if (i0 + 4 == N || chain_of<N8, N4, MODE>(P0 + i0 + 4) != hf) asm volatile("" : "+v"(rs[hf]));
   }
   asm volatile("" : "+v"(amax));
   return amax;
 }
 
 // Readout of segment sg: the sum of its chains.
-template <int N8, int N4>
+template <int N8, int N4, int MODE>
 __device__ __forceinline__ float segment_readout(int sg, const float (&rs)[8]) {
   const int last = seg_pos(N8, N4, sg + 1) - 1;
-  const bool second = half_of<N8, N4>(last) == 2 * sg + 1;
+  const bool second = chain_of<N8, N4, MODE>(last) == 2 * sg + 1;
   return second ? rs[2 * sg] + rs[2 * sg + 1] : rs[2 * sg];
 }
 
@@ -1398,9 +1406,9 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
             }
             fin8 = __builtin_fabsf(s8) <= 65504.f;
             if (__builtin_amdgcn_ballot_w64(!fin8) == 0)
-              amax8 = tier_update<M8, true, false, N8, N4, A8>(c8, s8, decay, x, bdt4, cw4, rs, v8);
+              amax8 = tier_update<M8, true, false, N8, N4, A8, MODE>(c8, s8, decay, x, bdt4, cw4, rs, v8);
             else
-              amax8 = tier_update<M8, true, true, N8, N4, A8>(c8, s8, decay, x, bdt4, cw4, rs, v8);
+              amax8 = tier_update<M8, true, true, N8, N4, A8, MODE>(c8, s8, decay, x, bdt4, cw4, rs, v8);
             if constexpr (SHARE8) pmax[0][R][lane] = amax8;
           }
           // the latent coefficients, read with the rows
@@ -1427,9 +1435,9 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
             }
             fin4 = __builtin_fabsf(s4) <= 65504.f;
             if (__builtin_amdgcn_ballot_w64(!fin4) == 0)
-              amax4 = tier_update<M4, false, false, N8, N4, N8 + A4>(c4, s4, decay, x, bdt4, cw4, rs, v4);
+              amax4 = tier_update<M4, false, false, N8, N4, N8 + A4, MODE>(c4, s4, decay, x, bdt4, cw4, rs, v4);
             else
-              amax4 = tier_update<M4, false, true, N8, N4, N8 + A4>(c4, s4, decay, x, bdt4, cw4, rs, v4);
+              amax4 = tier_update<M4, false, true, N8, N4, N8 + A4, MODE>(c4, s4, decay, x, bdt4, cw4, rs, v4);
             if constexpr (SHARE4) pmax[1][R][lane] = amax4;
           }
           uint32_t qz = 0;
@@ -1444,7 +1452,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           // the left fold of the readout segments: the other waves publish
           // the fold of their segments, the reading wave folds them in order
 #pragma unroll
-          for (int sg = G0; sg < G1; ++sg) accs[sg] = segment_readout<N8, N4>(sg, rs);
+          for (int sg = G0; sg < G1; ++sg) accs[sg] = segment_readout<N8, N4, MODE>(sg, rs);
           float part = accs[G0];
 #pragma unroll
           for (int sg = G0 + 1; sg < G1; ++sg) part = part + accs[sg];
@@ -1558,10 +1566,10 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
           {
             float v8[N8];
             if (__builtin_amdgcn_ballot_w64(!fin8) == 0) {
-              const float m8 = tier_update<N8, true, false, N8, N4, 0>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
+              const float m8 = tier_update<N8, true, false, N8, N4, 0, MODE>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
               sc8 = tier_requant<N8, true, MODE>(v8, c8, m8, base_ok);
             } else {
-              const float m8 = tier_update<N8, true, true, N8, N4, 0>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
+              const float m8 = tier_update<N8, true, true, N8, N4, 0, MODE>(c8, sc8, decay, x, bdt4, cw4, rs, v8);
               sc8 = tier_requant<N8, true, MODE>(v8, c8, m8, base_ok && fin8);
             }
           }
@@ -1609,10 +1617,10 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         {
           float v4[N4];
           if (__builtin_amdgcn_ballot_w64(!fin4) == 0) {
-            const float m4 = tier_update<N4, false, false, N8, N4, N8>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
+            const float m4 = tier_update<N4, false, false, N8, N4, N8, MODE>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
             sc4 = tier_requant<N4, false, MODE>(v4, c4, m4, base_ok);
           } else {
-            const float m4 = tier_update<N4, false, true, N8, N4, N8>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
+            const float m4 = tier_update<N4, false, true, N8, N4, N8, MODE>(c4, sc4, decay, x, bdt4, cw4, rs, v4);
             sc4 = tier_requant<N4, false, MODE>(v4, c4, m4, base_ok && fin4);
           }
         }
@@ -1622,7 +1630,7 @@ __device__ __forceinline__ void state_step_body(const StepArgs& a,
         __builtin_amdgcn_sched_barrier(0);
         float accs[4];
 #pragma unroll
-        for (int sg = 0; sg < 4; ++sg) accs[sg] = segment_readout<N8, N4>(sg, rs);
+        for (int sg = 0; sg < 4; ++sg) accs[sg] = segment_readout<N8, N4, MODE>(sg, rs);
         const float acc = ((accs[0] + accs[1]) + accs[2]) + accs[3];   // the readout segments' left fold
         // readout: sum_i u_i c_i + corrections = decay * (sum_i prior_i (c_i +
         // corr_i) + latent terms) + x * (dt * sum_all b c + D)
