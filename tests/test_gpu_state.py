@@ -776,6 +776,77 @@ def test_rows_scan_unusual_states(oracle, device, batch, L):
                nonfinite_y=True)
 
 
+def _scan_of(codec, device, batch, H, P):
+    """(state, scan(inputs, state, table)) of a codec whose scan is not the
+    ridge one."""
+    from mamba2_recall import state_codec, state_codec_dense3, tier_codec
+    if codec in ("legacy", "s16"):
+        return (state_codec.allocate_state(batch, H, P, 128, "sq3p25" if codec == "legacy" else "s16", device),
+                lambda a, st, table: state_codec.scan(*a, st, table if codec == "legacy" else None)[0])
+    if codec == "dense3":
+        return (state_codec_dense3.allocate_state(batch, H, P, 128, device),
+                lambda a, st, table: state_codec_dense3.scan(*a, st, table))
+    return (tier_codec.allocate_state(batch, H, P, 128, device, layout=codec),
+            lambda a, st, table: tier_codec.scan(*a, st, table, layout=codec)[0])
+
+
+@pytest.mark.parametrize("batch,L", [(1, 24), (5, 24), (8, 24), (13, 64)])
+@pytest.mark.parametrize("codec", ["legacy", "32_32_64", "8_80_40", "44_8_76", "dense3", "s16"])
+def test_tokens_and_batch_rows_in_one_call_or_many(device, codec, batch, L):
+    """One call of L tokens (the row-split scans on 8, 4, 2 and 1 or 4 lanes),
+    one call per token and one call per batch row, and a forced shape, give the
+    same state bit for bit and the same y to the order of a binary32 sum.  Two
+    such sums of 128 products differ by less than 2^-16 of the sum of their
+    magnitudes, here within 32 of y's norm, and then round to binary16: y
+    moves by one step, 2^-10 of it, where it moves at all."""
+    from mamba2_recall import _native
+    H, P, G = 128, 16, 8
+    print(f"[one call or many] codec={codec} B={batch} L={L}", flush=True)
+    rng = np.random.default_rng(batch * 100 + L)
+    inp = cases.step_inputs(rng, batch, L, H, P, G)
+    t = device_inputs(inp, device)
+    table = torch.from_numpy(inp["perm"]).to(device)
+
+    def fill(state, rows):
+        gen = torch.Generator(device=device).manual_seed(5)
+        for k, v in state.tensors.items():
+            shape = (batch,) + tuple(v.shape[1:])
+            if v.dtype == torch.float16:
+                new = torch.exp(torch.randn(shape, generator=gen, device=device) * 0.5 - 2.0).half()
+            else:
+                new = torch.randint(0, 256, shape, generator=gen, device=device, dtype=torch.uint8)
+            v.copy_(new[rows])
+
+    def run(pieces, shape=(0, 0)):
+        """`pieces`: (batch rows, tokens) slices, each batch row's tokens in order."""
+        ys, states = torch.empty_like(t["x"]), {}
+        for rows, runs in pieces:
+            n = len(range(*rows.indices(batch)))
+            state, scan = _scan_of(codec, device, n, H, P)
+            fill(state, rows)
+            _native.call("m2r_set_step_shape", *shape)
+            try:
+                for tok in runs:
+                    a = [t[k][rows, tok] for k in ("x", "dt")] + [t["A"]]
+                    a += [t[k][rows, tok] for k in ("B", "C")] + [t["D"], t["dt_bias"]]
+                    ys[rows, tok] = scan(a, state, table)
+            finally:
+                _native.call("m2r_set_step_shape", 0, 0)
+            for k, v in state.tensors.items():
+                states.setdefault(k, []).append(v)
+        return ys, {k: torch.cat(v) for k, v in states.items()}
+
+    everything, tokens = slice(0, batch), [slice(i, i + 1) for i in range(L)]
+    y0, s0 = run([(everything, [slice(0, L)])])
+    others = dict(tokens=run([(everything, tokens)]), forced=run([(everything, [slice(0, L)])], (4, 1)),
+                  rows=run([(slice(b, b + 1), [slice(0, L // 2), slice(L // 2, L)]) for b in range(batch)]))
+    for name, (y, s) in others.items():
+        for k in s0:
+            assert torch.equal(s[k].view(torch.uint8), s0[k].view(torch.uint8)), (name, k)
+        err = float((y.double() - y0.double()).norm() / y0.double().norm())
+        assert err <= 2.0 ** -10 + 2.0 ** -11, f"{name}: y rel L2 {err:.3e}"
+
+
 @pytest.mark.parametrize("batch,L", [(1, 24), (5, 24), (8, 24), (13, 64)])
 def test_rows_scan_stored_scales_overflow(oracle, device, batch, L):
     """A tier's stored scale that overflows binary16 from finite inputs, at a
