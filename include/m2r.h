@@ -116,7 +116,10 @@ int m2r_state_step_legacy(const void* x, const void* dt, const float* A, const v
  * slot (each wave steps a quarter of the carried coordinates); (0,0) restores
  * the automatic choice.  A forced shape whose head count does not divide the heads per group
  * falls back to the automatic choice.  A forced shape also keeps multi-token calls on the one-lane-per-row
- * kernels, with a ridge workspace too (which they do not use).  Process-wide; results do not depend on the shape.  No counterpart
+ * kernels, with a ridge workspace too (which they do not use).  Process-wide.  Codes, scales and latent
+ * bytes do not depend on the shape, nor does the ridge y.  The y of the other codecs agrees to the order of
+ * a binary32 sum between the multi-token scan and the one-lane kernels: it can differ in a last bit of FP16
+ * by the shape, and by how many tokens and batch rows a call takes.  No counterpart
  * in the reference (its Triton launch grid is fixed per call).
  */
 int m2r_set_step_shape(int waves_per_block, int heads_per_wave);
@@ -368,6 +371,8 @@ int m2r_gated_rmsnorm(const void* y, int64_t y_stride, const void* z, int64_t z_
  *   u_stride (16-byte aligned, u_stride % 8 == 0); y f16 rows of N with row
  *   stride y_stride.  M in {1, 2, 4}; K in {2048, 4096, 8192}.  The packet
  *   must satisfy the decode checks (no error word here).
+ * One and two rows give a row the same bits; four rows are summed in another
+ * order (matrix cores) where N >= 2,033 on 256 CUs, or K = 2048.
  */
 int m2r_fp4_gemv_g16(const uint8_t* packed, const uint8_t* e4m3_scales, const float* global_scale, const void* u,
                      int64_t u_stride, void* y, int64_t y_stride, int64_t M, int64_t N, int64_t K,

@@ -261,8 +261,8 @@ __global__ __launch_bounds__(64 * WPB) void k_fp4_gemv_rows(const uint8_t* __res
 }
 
 // Four activation rows: with a dot product per row and weight pair the vector
-// units have 3.4 instructions a weight, twice the 1.6 that form it, and the
-// sums of four rows; the matrix cores take the products and sums off them.  A
+// units have 3.75 instructions a weight, 1.75 of which form it, and the sums of
+// four rows; the matrix cores take the products and sums off them.  A
 // workgroup of NW waves takes tiles of 16 matrix rows, wave w the w-th part of
 // K, as v_mfma_f32_16x16x32_f16 with the 16 rows of weights (A) against the
 // four activation rows (B; the other 12 columns repeat the last one, unused).

@@ -29,13 +29,30 @@ inline long long rows_slots(long long B, int H, int P) { return B * H * ((P + 63
 
 // Lanes per row, by the scan's 64-row slots: enough to give every SIMD a
 // wave, then fewer, as each lane repeats a token's scalar work.  us for 64
-// tokens at batch 1, 3, 4, 8, 12, 16 and 64 (128 slots each), ridge 24/44/60:
-//   8 lanes   56.3   84.0  105.6  172.5  244.4  316.9
-//   4         78.7   90.6   91.7  155.2  198.0  255.0    923
-//   2        105.8  108.8  109.7  128.9  210.2  236.0    880
-//   1        162.2  164.2  164.0  174.5  196.3  203.4    753
-// One lane has all carried coordinates and updates in registers: with more
-// than 72 they spill (8/76/44 at batch 16: 279 against 273 on four lanes).
+// tokens on 8 / 4 / 2 / 1 lanes at batches of 128 slots each (records included):
+//                     3                 4               6               8
+//   ridge 24/44/60    77/ 81/ 98/154  110/ 86/100/155  143/108/115/159  177/129/118/161
+//   ridge 8/76/44     78/ 90/121      108/ 94/122      140/118/135      177/164/138
+//   tier 32/32/64     48/ 51/ 73/123   62/ 54/ 75/123   88/ 67/ 80/123  108/ 82/ 81/125
+//   tier 8/80/40      59/ 74/101       85/ 77/102      110/ 95/112      141/117/115
+//   legacy 16/64/48   55/ 64/ 85       79/ 66/ 86      104/ 85/ 97      134/105/ 99
+//   dense3            65/ 75/121       98/ 79/122      125/102/132      162/145/135
+//                     12               16              32              64
+//   ridge 24/44/60   249/177/148/179  321/222/204/185  -/410/344/352   -/791/649/690
+//   ridge 8/76/44    251/210/237      323/269/257      -/512/498       -/980/975
+//   tier 32/32/64    151/115/105/141  196/149/155/144  -/277/260/279   -/536/485/546
+//   tier 8/80/40     206/169/205      267/217/226      -/408/447       -/787/878
+//   legacy 16/64/48  193/148/129      253/193/184      -/357/311       -/696/591
+//   dense3           235/193/246      309/251/267      -/478/521       -/931/1039
+// The first three lines are where the order changes, within 3%, at every width
+// (batch 5 and 7 go the way of 6 and 8).  Past 1,024 slots the rule is coarser:
+// four lanes are right for 84 and more coordinates (within 5%), one lane for at
+// most 72 at 1,792 to 2,048 slots, but two lanes measure 1 to 17% faster than the
+// rule's for at most 72 at 1,280 and 1,536 slots, and 2 to 15% for some widths
+// beyond (24/44/60 and 32/32/64 from 4,096 slots, 16/60/52 from 1,792, 16/64/48 at
+// 1,536 and from 2,048).  One lane has all carried coordinates and updates in
+// registers: with more than 72 they spill (8/76/44 at batch 16: 279 against 273
+// on four lanes).
 inline int rows_lanes(int carried, long long slots) {
   if (slots <= 384) return 8;
   if (slots <= 768) return 4;
