@@ -206,9 +206,10 @@ hipError_t launch_s16_rows(const S16Args& a, hipStream_t stream) {
 // one-lane kernels: 8 heads in 8 groups at batch 500, 24 tokens, tier 32/32/64
 // 127 / 443.  A ridge scan's records serve the heads of a group: one head per
 // group pays from 64 tokens on to 1,280 slots (batch 138: 32 tokens 141 / 144, 64
-// 273 / 255), and not above (batch 175, 128 tokens 535 / 566); wide rows of two or
-// three heads to 1,536 (batch 122 of 9 heads, 64 tokens 294 / 214; batch 333 of 6,
-// 308 / 343).
+// 273 / 255), and not above (batch 175, 128 tokens 535 / 566).  Wide rows of two
+// or three heads per group gain from 64 tokens on almost everywhere (8/76/44, 16
+// heads in 8 groups of 16 rows at batch 345, 105 tokens 1,315 / 913; batch 122 of
+// 9 heads in 3, 64 tokens 294 / 214; a loss is batch 333 of 6 in 3, 308 / 343).
 int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int G) {
   const long long slots = rows_slots(B, H, P);
   const int lanes = rows_lanes(carried, slots), rows = 64 / lanes, hpg = H / G;
@@ -221,7 +222,7 @@ int rows_scan_lanes(int mode, int carried, long long B, int L, int H, int P, int
   if (mode == MODE_DENSE3) {
     least = slots <= 384 ? 2 : slots <= 1024 ? 4 : 16;
   } else if (mode == MODE_RIDGE) {
-    if (slots > (hpg == 1 ? 1280 : 1536) && hpg < (wide ? 4 : 2)) return 0;
+    if (slots > 1280 && hpg == 1) return 0;
     least = slots > 1024 && hpg == 1 ? 64 : slots <= 256 ? 16 : slots <= 384 ? 20 : slots <= 1024 ? (wide && slots > 768 ? 32 : 24) : wide ? 64 : 24;
   } else {
     if (!wide && carried > 52 && slots > 2048 && slots <= 3072) return 0;

@@ -78,7 +78,8 @@ def test_scan_lanes_leave_no_wave_without_rows():
     assert [lanes(TIER, 8, 80, b, 64, *model) for b in (1, 8, 16, 64)] == [8, 2, 4, 4]
     assert [lanes(TIER, 32, 32, b, 64, *model) for b in (17, 20, 24, 25)] == [0, 0, 0, 1]
     assert [lanes(TIER, 32, 32, b, 24, *model) for b in (16, 28, 32, 33)] == [1, 0, 1, 1]
-    assert lanes(TIER, 44, 8, 20, 24, *model) == 1 and lanes(RIDGE, 8, 76, 333, 64, 6, 64, 3) == 0
+    assert lanes(TIER, 44, 8, 20, 24, *model) == 1
+    assert [lanes(RIDGE, 8, 76, 345, L, 16, 16, 8) for L in (63, 64, 105)] == [0, 4, 4]
     assert [lanes(RIDGE, 24, 44, b, 32, 8, 64, 8) for b in (16, 100, 138, 175)] == [8, 0, 0, 0]
     assert lanes(RIDGE, 24, 44, 138, 64, 8, 64, 8) == 4 and lanes(RIDGE, 8, 76, 122, 64, 9, 64, 3) == 4
     assert [lanes(DENSE3, 0, 0, b, 16, *model) for b in (1, 4, 8, 64)] == [8, 4, 2, 4]
